@@ -35,6 +35,9 @@ _SIGS = {
     "attn_gemv_bias_residual": ([_P, _I64, _I64, _P, _I64, _P, _P, _P, _P], _INT),
     "attn_qkv_gemv_rope_append": ([_P, _I64, _I64, _P, _P, _F, _P, _P, _P, _P, _F, _P, _I64, _P,
                                    _P], _INT),
+    "attn_rows_bias_residual": ([_P, _I64, _I64, _P, _I64, _P, _P, _P, _P], _INT),
+    "attn_rows_qkv_rope_append": ([_P, _I64, _I64, _P, _P, _F, _P, _P, _P, _P, _F, _P, _I64, _P,
+                                   _P], _INT),
     "attn_sample_workspace_bytes": ([_I64], _SZ),
     "attn_sample_top_p": ([_P, _I64, _I64, _F, _F, _F, _P, _P, _SZ, _P], _INT),
 }
@@ -216,9 +219,7 @@ def gemv(x: torch.Tensor, W: torch.Tensor, out: torch.Tensor | None = None,
     return out
 
 
-def gemv_bias_residual(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor,
-                       residual: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
-    """bf16(residual + bf16(bf16(x @ W^T) + bias)) for at most 8 token rows."""
+def _bias_residual_fused(fn, what, x, W, bias, residual, out):
     _expect(x, "x", torch.bfloat16)
     _expect(W, "W", torch.bfloat16)
     N, K = W.shape
@@ -230,17 +231,19 @@ def gemv_bias_residual(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor,
     if out is None:
         out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     _expect(out, "out", torch.bfloat16)
-    _check(_lib.attn_gemv_bias_residual(_ptr(x), M, K, _ptr(W), N, _ptr(bias), _ptr(residual),
-                                        _ptr(out), _stream()), "attn_gemv_bias_residual")
+    _check(fn(_ptr(x), M, K, _ptr(W), N, _ptr(bias), _ptr(residual), _ptr(out), _stream()), what)
     return out
 
 
-def qkv_gemv_rope_append(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor,
-                         positions: torch.Tensor, slots: torch.Tensor, inv_freq: torch.Tensor,
-                         concentration: float, kv_cache: torch.Tensor, q_out: torch.Tensor,
-                         norm_w: torch.Tensor | None = None, eps: float = 1e-5) -> torch.Tensor:
-    """The decode QKV projection with bias, RoPE and the cache append fused
-    (and the block's pre-norm when norm_w is given)."""
+def gemv_bias_residual(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor,
+                       residual: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+    """bf16(residual + bf16(bf16(x @ W^T) + bias)) for at most 8 token rows."""
+    return _bias_residual_fused(_lib.attn_gemv_bias_residual, "attn_gemv_bias_residual", x, W,
+                                bias, residual, out)
+
+
+def _qkv_fused(fn, what, x, W, bias, positions, slots, inv_freq, concentration, kv_cache, q_out,
+               norm_w, eps):
     _expect(x, "x", torch.bfloat16)
     _expect(W, "W", torch.bfloat16)
     N, K = W.shape
@@ -255,9 +258,36 @@ def qkv_gemv_rope_append(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor,
     _expect(q_out, "q_out", torch.bfloat16, (M, Q_HEADS, HEAD_DIM))
     if norm_w is not None:
         _expect(norm_w, "norm_w", torch.bfloat16, (K,))
-    _check(_lib.attn_qkv_gemv_rope_append(_ptr(x), M, K, _ptr(W), _ptr(norm_w), eps, _ptr(bias),
-                                          _ptr(positions),
-                                          _ptr(slots), _ptr(inv_freq), concentration,
-                                          _ptr(kv_cache), kv_cache.shape[0], _ptr(q_out),
-                                          _stream()), "attn_qkv_gemv_rope_append")
+    _check(fn(_ptr(x), M, K, _ptr(W), _ptr(norm_w), eps, _ptr(bias), _ptr(positions), _ptr(slots),
+              _ptr(inv_freq), concentration, _ptr(kv_cache), kv_cache.shape[0], _ptr(q_out),
+              _stream()), what)
     return q_out
+
+
+def qkv_gemv_rope_append(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor,
+                         positions: torch.Tensor, slots: torch.Tensor, inv_freq: torch.Tensor,
+                         concentration: float, kv_cache: torch.Tensor, q_out: torch.Tensor,
+                         norm_w: torch.Tensor | None = None, eps: float = 1e-5) -> torch.Tensor:
+    """The decode QKV projection with bias, RoPE and the cache append fused
+    (and the block's pre-norm when norm_w is given)."""
+    return _qkv_fused(_lib.attn_qkv_gemv_rope_append, "attn_qkv_gemv_rope_append", x, W, bias,
+                      positions, slots, inv_freq, concentration, kv_cache, q_out, norm_w, eps)
+
+
+ROWS_MAX_TOKENS = 16
+
+
+def rows_bias_residual(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor,
+                       residual: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+    """gemv_bias_residual for at most 16 token rows."""
+    return _bias_residual_fused(_lib.attn_rows_bias_residual, "attn_rows_bias_residual", x, W,
+                                bias, residual, out)
+
+
+def rows_qkv_rope_append(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor,
+                         positions: torch.Tensor, slots: torch.Tensor, inv_freq: torch.Tensor,
+                         concentration: float, kv_cache: torch.Tensor, q_out: torch.Tensor,
+                         norm_w: torch.Tensor | None = None, eps: float = 1e-5) -> torch.Tensor:
+    """qkv_gemv_rope_append for at most 16 token rows."""
+    return _qkv_fused(_lib.attn_rows_qkv_rope_append, "attn_rows_qkv_rope_append", x, W, bias,
+                      positions, slots, inv_freq, concentration, kv_cache, q_out, norm_w, eps)

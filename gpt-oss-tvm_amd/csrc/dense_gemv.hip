@@ -1,16 +1,16 @@
-// Decode-sized dense projections of the gpt-oss layer (M <= 8 tokens): the
-// fused QKV nn.Linear with its bias, YaRN RoPE and the KV-cache append; the
+// Dense projections of the gpt-oss layer for one token (dense_rows.hip takes
+// two and more): the fused QKV nn.Linear with its bias, YaRN RoPE and the KV-cache append; the
 // attention output nn.Linear with its bias and the residual add; the
 // unembedding (model/attention.py:204,254-256; model/transformer.py:95-100).
 // The QKV projection and the unembedding can also apply the RMSNorm before
 // them (attention.py:80, transformer.py:63) to the rows they stage.
 //
-// y[m][n] = sum_k x[m][k] W[n][k], bf16 operands, fp32 accumulation, one bf16
+// y[n] = sum_k x[k] W[n][k], bf16 operands, fp32 accumulation, one bf16
 // rounding (the matmul's output dtype), then the epilogue's own bf16 ops.
 // HBM-bound on W.  A workgroup takes RW rows of W; its 4 waves split K (wave
 // w takes the 16-byte chunks w * 64 + lane + 256 i of each row), so a row's
 // bytes stream from four waves at once; the four partial sums are added in
-// wave order through LDS (deterministic).  The tokens x are staged in LDS.
+// wave order through LDS (deterministic).  The token x is staged in LDS.
 // Loads complete in issue order, so everything small that the workgroup
 // needs (its x chunks, the epilogue's bias, residual, positions, slots and
 // RoPE frequencies) is loaded before the W rows, and the epilogue's cos and
@@ -26,7 +26,6 @@ using moe::u32x4;
 
 constexpr int kThreads = 256;  // 4 waves
 constexpr int kWaves = 4;
-constexpr int kMaxM = 8;
 constexpr int kIters = 2;  // 16-byte chunk rounds per lane: K <= 4096 = 2 x 256 x 8
 
 // gpt-oss attention shapes (the QKV epilogue)
@@ -47,7 +46,7 @@ enum Epi { kPlain = 0, kBiasResidual = 1, kQkv = 2 };
 
 struct Args {
   const uint16_t* x;
-  int M, K;
+  int K;
   const uint16_t* W;
   int N;
   uint16_t* out;
@@ -65,14 +64,14 @@ struct Args {
   uint16_t* q_out;
 };
 
-template <int RW, int EPI, int MM>
+template <int RW, int EPI>
 __global__ __launch_bounds__(kThreads) void gemv_kernel(Args a) {
 #pragma clang fp contract(off)
-  extern __shared__ __align__(16) uint16_t xs[];  // the M token rows, M * K bf16
-  __shared__ float part[kWaves][RW][kMaxM];
-  __shared__ double ssq[kWaves][kMaxM];
+  extern __shared__ __align__(16) uint16_t xs[];  // the token's row, K bf16
+  __shared__ float part[kWaves][RW];
+  __shared__ double ssq[kWaves];
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const int M = a.M, K = a.K, N = a.N;
+  const int K = a.K, N = a.N;
   const int chunks = K / 8;
   // this workgroup's rows
   int rows[RW];
@@ -90,8 +89,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(Args a) {
 #pragma unroll
     for (int i = 0; i < RW; ++i) rows[i] = blockIdx.x * RW + i;
   }
-  // x's chunks of this thread (one token: at eight, holding them would cost
-  // occupancy) and the epilogue's operands first (they are needed first),
+  // x's chunks of this thread and the epilogue's operands first (they are needed first),
   // then every W load of this lane (K <= 4096: at most two rounds of 256
   // 16-byte chunks) with the norm weight's chunks when the rows are
   // normalised.  Every load is unconditional (indices clamped into range,
@@ -101,30 +99,27 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(Args a) {
   // between them.
   const bool norm = a.norm_w != nullptr;
   const uint16_t* const nw = norm ? a.norm_w : a.W;  // (loaded, unused, without a norm)
-  constexpr bool kEarlyX = MM == 1;
-  u32x4 xr[kEarlyX ? 1 : 0 + 1][kIters];
-  if constexpr (kEarlyX) {
+  u32x4 xr[kIters];
 #pragma unroll
-    for (int it = 0; it < kIters; ++it)
-      xr[0][it] = *(const u32x4*)(a.x + min(it * kThreads + t, chunks - 1) * 8);
-  }
-  // the epilogue task of this thread (one per row or rope pair, and token)
+  for (int it = 0; it < kIters; ++it)
+    xr[it] = *(const u32x4*)(a.x + min(it * kThreads + t, chunks - 1) * 8);
+  // the epilogue task of this thread (one per row or rope pair)
   constexpr int kTasks = EPI == kQkv ? RW / 2 : RW;
-  const bool task = t < kTasks * M;
-  const int ti = task ? t / M : 0, tm = task ? t % M : 0;
+  const bool task = t < kTasks;
+  const int ti = task ? t : 0;
   uint16_t eb0r = 0, eb1r = 0, err = 0;
   float cs = 0.f, sn = 0.f, ifq = 0.f;
   int eslot = -1, epos = 0;
   if constexpr (EPI == kBiasResidual) {
     const int n = min(rows[ti], N - 1);
     eb0r = a.bias[n];
-    err = a.res[(size_t)tm * N + n];
+    err = a.res[n];
   } else if constexpr (EPI == kQkv) {
     const int nlo = rows[2 * ti], nhi = rows[2 * ti + 1];
     eb0r = a.bias[nlo];
     eb1r = a.bias[nhi];
-    eslot = a.slots[tm];
-    epos = a.positions[tm];
+    eslot = a.slots[0];
+    epos = a.positions[0];
     ifq = a.inv_freq[nlo % kD];
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -143,101 +138,81 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(Args a) {
   if constexpr (EPI == kQkv) {
     if (task && rows[2 * ti] / kD < kHq + kHkv) {
       const float freq = (float)epos * ifq;
-      const double fd = (double)freq;
-      cs = bf2f(f2bf((float)cos(fd))) * a.conc;
-      sn = bf2f(f2bf((float)sin(fd))) * a.conc;
+      double sd, cd;
+      moe::sincos_f64((double)freq, sd, cd);
+      cs = bf2f(moe::f64_to_bf16_via_f32(cd)) * a.conc;
+      sn = bf2f(moe::f64_to_bf16_via_f32(sd)) * a.conc;
     }
   }
   // Stage x; for the RMSNorm, the sum of squares of the bf16 values in fp64
-  // (exact for rows spanning less than 2^37) on the way, as the standalone
+  // (exact for a row spanning less than 2^37) on the way, as the standalone
   // kernel: r = fp32(1 / sqrt(ss / K + eps)), t = bf16(fp32(x r) w)
+  double ss = 0.0;
 #pragma unroll
-  for (int m = 0; m < MM; ++m) {
-    if (m >= M) break;
-    double ss = 0.0;
+  for (int it = 0; it < kIters; ++it) {
+    const int c = it * kThreads + t;
+    if (c >= chunks) continue;
+    const u32x4 v = xr[it];
+    *(u32x4*)(xs + c * 8) = v;
+    if (norm) {
 #pragma unroll
-    for (int it = 0; it < kIters; ++it) {
-      const int c = it * kThreads + t;
-      if (c >= chunks) continue;
-      const u32x4 v = kEarlyX ? xr[0][it] : *(const u32x4*)(a.x + (size_t)m * K + c * 8);
-      *(u32x4*)(xs + m * K + c * 8) = v;
-      if (norm) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const double lo = (double)__uint_as_float(v[j] << 16);
-          const double hi = (double)__uint_as_float(v[j] & 0xFFFF0000u);
-          ss += lo * lo + hi * hi;
-        }
+      for (int j = 0; j < 4; ++j) {
+        const double lo = (double)__uint_as_float(v[j] << 16);
+        const double hi = (double)__uint_as_float(v[j] & 0xFFFF0000u);
+        ss += lo * lo + hi * hi;
       }
     }
-    if (norm) {
-      ss = moe::wave_sum(ss);
-      if (lane == 0) ssq[wave][m] = ss;
-    }
+  }
+  if (norm) {
+    ss = moe::wave_sum(ss);
+    if (lane == 0) ssq[wave] = ss;
   }
   __syncthreads();
-  float rn[MM];
-#pragma unroll
-  for (int m = 0; m < MM; ++m) {
-    rn[m] = 1.0f;
-    if (norm && m < M) {
-      const double tot = (ssq[0][m] + ssq[1][m]) + (ssq[2][m] + ssq[3][m]);
-      rn[m] = (float)(1.0 / sqrt(tot / (double)K + (double)a.eps));
-    }
+  float rn = 1.0f;
+  if (norm) {
+    const double tot = (ssq[0] + ssq[1]) + (ssq[2] + ssq[3]);
+    rn = (float)(1.0 / sqrt(tot / (double)K + (double)a.eps));
   }
-  float acc[RW][MM];
+  float acc[RW];
 #pragma unroll
-  for (int i = 0; i < RW; ++i)
-#pragma unroll
-    for (int m = 0; m < MM; ++m) acc[i][m] = 0.f;
+  for (int i = 0; i < RW; ++i) acc[i] = 0.f;
 #pragma unroll
   for (int it = 0; it < kIters; ++it) {
     const int c = it * kThreads + wave * 64 + lane;
     if (c < chunks) {
+      u32x4 xv = *(const u32x4*)(xs + c * 8);
+      if (norm) {
 #pragma unroll
-      for (int m = 0; m < MM; ++m) {
-        if (m < M) {
-          u32x4 xv = *(const u32x4*)(xs + m * K + c * 8);
-          if (norm) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const uint32_t lo = f2bf(__fmul_rn(__fmul_rn(__uint_as_float(xv[j] << 16), rn[m]),
-                                                 __uint_as_float(nwv[it][j] << 16)));
-              const uint32_t hi = f2bf(__fmul_rn(__fmul_rn(__uint_as_float(xv[j] & 0xFFFF0000u),
-                                                           rn[m]),
-                                                 __uint_as_float(nwv[it][j] & 0xFFFF0000u)));
-              xv[j] = lo | (hi << 16);
-            }
-          }
-#pragma unroll
-          for (int i = 0; i < RW; ++i) acc[i][m] = dot8(wv[it][i], xv, acc[i][m]);
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t lo = f2bf(__fmul_rn(__fmul_rn(__uint_as_float(xv[j] << 16), rn),
+                                             __uint_as_float(nwv[it][j] << 16)));
+          const uint32_t hi = f2bf(__fmul_rn(__fmul_rn(__uint_as_float(xv[j] & 0xFFFF0000u), rn),
+                                             __uint_as_float(nwv[it][j] & 0xFFFF0000u)));
+          xv[j] = lo | (hi << 16);
         }
       }
+#pragma unroll
+      for (int i = 0; i < RW; ++i) acc[i] = dot8(wv[it][i], xv, acc[i]);
     }
   }
 #pragma unroll
-  for (int i = 0; i < RW; ++i)
-#pragma unroll
-    for (int m = 0; m < MM; ++m)
-      if (m < M) {
-        const float v = moe::wave_sum(acc[i][m]);
-        if (lane == 0) part[wave][i][m] = v;
-      }
+  for (int i = 0; i < RW; ++i) {
+    const float v = moe::wave_sum(acc[i]);
+    if (lane == 0) part[wave][i] = v;
+  }
   __syncthreads();
-  // epilogue: one thread per (row or rope pair, token); partials in wave order
-  auto total = [&](int i, int m) {
-    return ((part[0][i][m] + part[1][i][m]) + part[2][i][m]) + part[3][i][m];
-  };
+  // epilogue: one thread per row or rope pair; partials in wave order
+  auto total = [&](int i) { return ((part[0][i] + part[1][i]) + part[2][i]) + part[3][i]; };
   if constexpr (EPI == kPlain || EPI == kBiasResidual) {
     if (task) {
-      const int i = ti, m = tm, n = rows[i];
+      const int n = rows[ti];
       if (n < N) {
-        const uint16_t y = f2bf(total(i, m));
+        const uint16_t y = f2bf(total(ti));
         if constexpr (EPI == kPlain) {
-          a.out[(size_t)m * N + n] = y;
+          a.out[n] = y;
         } else {
           const float tb = bf2f(f2bf(bf2f(y) + bf2f(eb0r)));
-          a.out[(size_t)m * N + n] = f2bf(bf2f(err) + tb);
+          a.out[n] = f2bf(bf2f(err) + tb);
         }
       }
     }
@@ -245,11 +220,10 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(Args a) {
     // bias (its own bf16 rounding), then YaRN RoPE of q / k heads exactly as
     // the standalone append kernel does, then q out or the cache slot
     if (task) {
-      const int i = ti, m = tm;
-      const int nlo = rows[2 * i];
+      const int nlo = rows[2 * ti];
       const int head = nlo / kD, d = nlo % kD;
-      float lo = bf2f(f2bf(bf2f(f2bf(total(2 * i, m))) + bf2f(eb0r)));
-      float hi = bf2f(f2bf(bf2f(f2bf(total(2 * i + 1, m))) + bf2f(eb1r)));
+      float lo = bf2f(f2bf(bf2f(f2bf(total(2 * ti))) + bf2f(eb0r)));
+      float hi = bf2f(f2bf(bf2f(f2bf(total(2 * ti + 1))) + bf2f(eb1r)));
       if (head < kHq + kHkv) {
         const float nl = lo * cs - hi * sn;
         const float nh = lo * sn + hi * cs;
@@ -259,7 +233,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(Args a) {
       const uint16_t blo = f2bf(lo), bhi = f2bf(hi);
       const int slot = eslot;
       if (head < kHq) {
-        uint16_t* qo = a.q_out + ((size_t)m * kHq + head) * kD;
+        uint16_t* qo = a.q_out + (size_t)head * kD;
         qo[d] = blo;
         qo[d + 32] = bhi;
       } else if (slot >= 0 && slot < a.num_pages * kPage) {
@@ -279,13 +253,11 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(Args a) {
 
 extern "C" {
 
-int attn_launch_gemv(const void* x, int M, int K, const void* W, int N, void* out,
-                     const void* norm_w, float eps, const void* bias, const void* res,
-                     hipStream_t s) {
+int attn_launch_gemv(const void* x, int K, const void* W, int N, void* out, const void* norm_w,
+                     float eps, const void* bias, const void* res, hipStream_t s) {
   using namespace gemv;
   Args a{};
   a.x = (const uint16_t*)x;
-  a.M = M;
   a.K = K;
   a.W = (const uint16_t*)W;
   a.N = N;
@@ -294,29 +266,21 @@ int attn_launch_gemv(const void* x, int M, int K, const void* W, int N, void* ou
   a.eps = eps;
   a.bias = (const uint16_t*)bias;
   a.res = (const uint16_t*)res;
-  const size_t lds = (size_t)M * K * 2;
-  // one token (batch-1 decode): accumulators for one row of x only
+  const size_t lds = (size_t)K * 2;
   if (bias) {
     constexpr int RW = 4;
-    const dim3 grid((N + RW - 1) / RW);
-    if (M == 1)
-      hipLaunchKernelGGL((gemv_kernel<RW, kBiasResidual, 1>), grid, dim3(kThreads), lds, s, a);
-    else
-      hipLaunchKernelGGL((gemv_kernel<RW, kBiasResidual, kMaxM>), grid, dim3(kThreads), lds, s, a);
-  } else if (M == 1) {
-    constexpr int RW = 16;
-    hipLaunchKernelGGL((gemv_kernel<RW, kPlain, 1>), dim3((N + RW - 1) / RW), dim3(kThreads), lds,
-                       s, a);
-  } else {
-    constexpr int RW = 8;
-    hipLaunchKernelGGL((gemv_kernel<RW, kPlain, kMaxM>), dim3((N + RW - 1) / RW), dim3(kThreads),
+    hipLaunchKernelGGL((gemv_kernel<RW, kBiasResidual>), dim3((N + RW - 1) / RW), dim3(kThreads),
                        lds, s, a);
+  } else {
+    constexpr int RW = 16;
+    hipLaunchKernelGGL((gemv_kernel<RW, kPlain>), dim3((N + RW - 1) / RW), dim3(kThreads), lds, s,
+                       a);
   }
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 
-int attn_launch_qkv_gemv(const void* x, int M, int K, const void* W, const void* norm_w,
-                         float eps, const void* bias, const int* positions, const int* slots,
+int attn_launch_qkv_gemv(const void* x, int K, const void* W, const void* norm_w, float eps,
+                         const void* bias, const int* positions, const int* slots,
                          const float* inv_freq, float conc, void* cache, int num_pages,
                          void* q_out, hipStream_t s) {
   using namespace gemv;
@@ -324,7 +288,6 @@ int attn_launch_qkv_gemv(const void* x, int M, int K, const void* W, const void*
   constexpr int RW = 4;  // two rope pairs per workgroup
   Args a{};
   a.x = (const uint16_t*)x;
-  a.M = M;
   a.K = K;
   a.W = (const uint16_t*)W;
   a.N = heads * kD;
@@ -338,12 +301,8 @@ int attn_launch_qkv_gemv(const void* x, int M, int K, const void* W, const void*
   a.cache = (uint8_t*)cache;
   a.num_pages = num_pages;
   a.q_out = (uint16_t*)q_out;
-  const dim3 grid(heads * (32 / (RW / 2)));
-  if (M == 1)
-    hipLaunchKernelGGL((gemv_kernel<RW, kQkv, 1>), grid, dim3(kThreads), (size_t)K * 2, s, a);
-  else
-    hipLaunchKernelGGL((gemv_kernel<RW, kQkv, kMaxM>), grid, dim3(kThreads), (size_t)M * K * 2, s,
-                       a);
+  hipLaunchKernelGGL((gemv_kernel<RW, kQkv>), dim3(heads * (32 / (RW / 2))), dim3(kThreads),
+                     (size_t)K * 2, s, a);
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 

@@ -1,0 +1,389 @@
+// Dense projections for 2 to 16 token rows on the bf16 matrix cores: the
+// fused QKV nn.Linear with its bias, YaRN RoPE and the KV-cache append; the
+// attention output nn.Linear with its bias and the residual add; the
+// unembedding (model/attention.py:204,254-256; model/transformer.py:95-100).
+//
+// y[m][n] = sum_k t[m][k] W[n][k], bf16 operands, fp32 accumulation, one bf16
+// rounding, then the epilogue's own bf16 ops, as dense_gemv.hip (one token)
+// does.  Bound by the bytes of W: a vector dot product per (row, token) is
+// issue-bound from two tokens on, while the matrix cores multiply 16 W rows by
+// 16 tokens for the price of the loads: the 201088 x 2880 unembedding at 2, 5
+// and 8 tokens 399, 750 and 1122 us on the vector ALUs, 198-201 here (5.8 TB/s);
+// QKV with its norm at 2 and 8 tokens 19.1 and 54.1 us, 12.2-12.6 here; the output
+// projection 10.6 and 34.1, 7.9-8.7 here.  (One token stays on the vector ALUs:
+// 9.1 and 6.5 us.)
+//
+// A workgroup takes 16 or 32 rows of W at a time; its sixteen waves split K
+// into contiguous runs of 32-wide steps (5 or 6 each at K = 2880), so that
+// every byte of the rows is in flight at once, and add their partial tiles
+// through LDS in fp64 (deterministic, one rounding).  v_mfma_f32_16x16x32_bf16: lane (r, g) =
+// (l % 16, l / 16) gives A row r (a W row) and B column r (a token), k = 8 g ..
+// 8 g + 7 of the step for both; D element i of the lane is W row 4 g + i,
+// token r.  Neither operand goes through LDS: a wave's K run of W and of the
+// tokens is used by that wave alone.
+// The tokens stay in registers (kSteps x 16 bytes a lane); for the unembedding a
+// workgroup walks a contiguous range of row groups with two groups' W in
+// flight.  The RMSNorm is the standalone kernel's arithmetic: the sum of squares
+// in fp64 from the lanes' own chunks.
+#include "moe_common.h"
+
+namespace rows {
+
+using moe::as_bf16x8;
+using moe::bf2f;
+using moe::f2bf;
+using moe::f32x4;
+using moe::kWave;
+using moe::u32x4;
+
+constexpr int kWaves = 16;
+constexpr int kThreads = kWaves * kWave;
+constexpr int kMaxGroups = 64;  // row groups of one workgroup's range (its outputs wait in LDS)
+
+// gpt-oss attention shapes (the QKV epilogue)
+constexpr int kD = 64, kHq = 64, kHkv = 8, kPage = 16;
+constexpr int kHeadBlock = kPage * kD * 2;
+constexpr int kPageBytes = 2 * kHkv * kHeadBlock;
+
+enum Epi { kPlain = 0, kBiasResidual = 1, kQkv = 2 };
+
+struct Args {
+  const uint16_t* x;
+  int M, K;
+  const uint16_t* W;
+  int N;
+  uint16_t* out;
+  const uint16_t* norm_w;
+  float eps;
+  const uint16_t* bias;
+  const uint16_t* res;
+  // QKV epilogue
+  const int* positions;
+  const int* slots;
+  const float* inv_freq;
+  float conc;
+  uint8_t* cache;
+  int num_pages;
+  uint16_t* q_out;
+};
+
+// The W row of A row `r` of row group `group`.  QKV: eight rope pairs, a
+// pair's two dimensions in one lane's result: A rows 4 g + i hold dimensions
+// d0 + 2 g + i % 2 + 32 (i / 2) of a head.
+template <int EPI>
+__device__ __forceinline__ int w_row(int group, int r) {
+  if constexpr (EPI == kQkv)
+    return (group >> 2) * kD + (group & 3) * 8 + 2 * (r >> 2) + (r & 1) + 32 * ((r >> 1) & 1);
+  else
+    return group * 16 + r;
+}
+
+// kSteps: 32-wide steps of K a wave holds (at most); kNorm: RMSNorm the tokens
+// first.  Row groups of a workgroup: a range walked two at a time (kPlain), two
+// (kQkv: 160 workgroups, all resident at once; with one group each the 320 ran
+// in two rounds) or one.
+template <int kSteps, int EPI, bool kNorm>
+__global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
+#pragma clang fp contract(off)
+  constexpr bool kTwo = EPI != kBiasResidual;  // two row groups in flight
+  constexpr int kRg = EPI == kQkv ? 2 : 1;     // row groups of a workgroup (kPlain: a range)
+  // partial tiles: of the two groups, or (kPlain) of the current and the last
+  __shared__ __align__(16) double part[kWaves][kTwo ? 2 : 1][4][kWave];
+  __shared__ double ssq[kWaves][16];
+  extern __shared__ __align__(16) uint16_t outs[];  // kPlain: [M][16 row groups of the range]
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int M = a.M, K = a.K, N = a.N;
+  const int steps = (K + 31) / 32;
+  const int s0 = steps * wave / kWaves;
+  const int cnt = steps * (wave + 1) / kWaves - s0;
+  // Lane's k of the wave's step s; steps past the wave's run and chunks past K
+  // read clamped addresses and count as zeros (in both operands).
+  auto k_of = [&](int s) { return (s0 + s) * 32 + 8 * g; };
+  auto valid = [&](int s) { return s < cnt && k_of(s) < K; };
+  auto load = [&](const uint16_t* row, int s) {
+    return *(const u32x4*)(row + min(k_of(s), K - 8));
+  };
+  const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
+  // this workgroup's row groups
+  int grp0 = blockIdx.x * kRg, grp1 = grp0 + kRg;
+  if constexpr (EPI == kPlain) {
+    const int64_t groups = (N + 15) / 16;
+    grp0 = (int)(groups * blockIdx.x / gridDim.x);
+    grp1 = (int)(groups * (blockIdx.x + 1) / gridDim.x);
+  }
+
+  // Issue order: the tokens, the epilogue's operands, then W (loads complete
+  // in issue order, and the norm and RoPE factors are taken while W streams).
+  u32x4 xf[kSteps];
+  {
+    const uint16_t* row = a.x + (size_t)min(r, M - 1) * K;
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) xf[s] = load(row, s);
+  }
+  // The epilogue task of waves 0..3, token r: element `wave` of a lane's four
+  // (W row 4 g + wave), or for QKV of row group wave / 2 the rope pair wave % 2 of
+  // the lane's two (elements j and j + 2).
+  const bool task = wave < 4 && r < M;
+  const int tm = min(r, M - 1);
+  const int tgrp = grp0 + (EPI == kQkv ? (wave >> 1) & 1 : 0);
+  const int ei = EPI == kQkv ? wave & 1 : wave & 3;
+  uint16_t eb0 = 0, eb1 = 0, er = 0;
+  float ifq = 0.f, cs = 0.f, sn = 0.f;
+  int eslot = -1, epos = 0, erow = 0;
+  if constexpr (EPI != kPlain) {
+    erow = min(w_row<EPI>(tgrp, 4 * g + ei), N - 1);
+    eb0 = a.bias[erow];
+    if constexpr (EPI == kBiasResidual) er = a.res[(size_t)tm * N + erow];
+  }
+  if constexpr (EPI == kQkv) {
+    eb1 = a.bias[erow + 32];
+    eslot = a.slots[tm];
+    epos = a.positions[tm];
+    ifq = a.inv_freq[erow % kD];
+  }
+  u32x4 nw[kNorm ? kSteps : 1];
+  if constexpr (kNorm) {
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) nw[s] = load(a.norm_w, s);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  u32x4 wa[kSteps], wb[kTwo ? kSteps : 1];
+  auto load_w = [&](auto& dst, int group) {
+    const uint16_t* row = a.W + (size_t)min(w_row<EPI>(group, r), N - 1) * K;
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) dst[s] = load(row, s);
+  };
+  load_w(wa, min(grp0, grp1 - 1));
+  // (behind the norm, whose weights hold registers until then)
+  if constexpr (kTwo && !kNorm) load_w(wb, min(grp0 + 1, grp1 - 1));
+  __builtin_amdgcn_sched_barrier(0);
+
+  if constexpr (EPI == kQkv) {  // the RoPE factors while W streams
+    if (task && erow / kD < kHq + kHkv) {
+      double sd, cd;
+      moe::sincos_f64((double)((float)epos * ifq), sd, cd);
+      cs = bf2f(moe::f64_to_bf16_via_f32(cd)) * a.conc;
+      sn = bf2f(moe::f64_to_bf16_via_f32(sd)) * a.conc;
+    }
+  }
+  if constexpr (kNorm) {
+    // r = fp32(1 / sqrt(sum of squares / K + eps)), t = bf16(fp32(x r) w)
+    double ss = 0.0;
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      const u32x4 v = valid(s) ? xf[s] : zero;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const double lo = (double)__uint_as_float(v[j] << 16);
+        const double hi = (double)__uint_as_float(v[j] & 0xFFFF0000u);
+        ss += lo * lo + hi * hi;
+      }
+    }
+    ss += __shfl_xor(ss, 16, kWave);
+    ss += __shfl_xor(ss, 32, kWave);
+    if (g == 0) ssq[wave][r] = ss;
+    moe::lds_barrier();
+    double tot = 0.0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) tot += ssq[w][r];
+    const float rn = (float)(1.0 / sqrt(tot / (double)K + (double)a.eps));
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t v = xf[s][j], w = nw[s][j];
+        const uint32_t lo = f2bf(__fmul_rn(__fmul_rn(__uint_as_float(v << 16), rn),
+                                           __uint_as_float(w << 16)));
+        const uint32_t hi = f2bf(__fmul_rn(__fmul_rn(__uint_as_float(v & 0xFFFF0000u), rn),
+                                           __uint_as_float(w & 0xFFFF0000u)));
+        xf[s][j] = lo | (hi << 16);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kTwo) load_w(wb, min(grp0 + 1, grp1 - 1));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  auto zero_tail = [&](u32x4 (&v)[kSteps]) {
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) v[s] = valid(s) ? v[s] : zero;
+  };
+  // One wave's partial tile of the loaded W rows, into LDS.  It is summed in
+  // fp64 after every two MFMAs (64 products): chained in fp32 over the wave's
+  // steps, 110 to 145 of a million results at K = 4096 rounded to the other bf16
+  // neighbour of a near tie, against 90 to 97 for the vector ALUs' short chains
+  // and 55 to 94 this way.
+  auto products = [&](const u32x4 (&w)[kSteps], int tile) {
+    double sum[4] = {};
+#pragma unroll
+    for (int s = 0; s < kSteps; s += 2) {
+      f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+      acc = moe::mfma16x16x32(as_bf16x8(w[s]), as_bf16x8(xf[s]), acc);
+      acc = moe::mfma16x16x32(as_bf16x8(w[s + 1]), as_bf16x8(xf[s + 1]), acc);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum[i] += (double)acc[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) part[wave][tile][i][lane] = sum[i];
+  };
+  // element i of this lane's four of a tile: the waves' partials added in fp64
+  // and rounded once
+  auto total = [&](int tile, int i) {
+    double v = part[0][tile][i][lane];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) v += part[w][tile][i][lane];
+    return (float)v;
+  };
+
+  if constexpr (EPI == kPlain) {
+    zero_tail(xf);
+    const int width = 16 * (grp1 - grp0);
+    // a row group: products, then the group after next takes the W registers'
+    // place in flight, and waves 0..3 sum one element of a lane's four each
+    // into the LDS outputs (buf alternates: a buffer is written again only
+    // after the next round's barrier, which follows its reads)
+    auto round = [&](u32x4 (&w)[kSteps], int group, int buf) {
+      zero_tail(w);
+      products(w, buf);
+      __builtin_amdgcn_sched_barrier(0);
+      load_w(w, min(group + 2, grp1 - 1));
+      __builtin_amdgcn_sched_barrier(0);
+      moe::lds_barrier();
+      if (task) outs[r * width + 16 * (group - grp0) + 4 * g + ei] = f2bf(total(buf, ei));
+    };
+    int group = grp0;
+    for (; group + 1 < grp1; group += 2) {
+      round(wa, group, 0);
+      round(wb, group + 1, 1);
+    }
+    if (group < grp1) round(wa, group, 0);
+    moe::lds_barrier();
+    // the range's outputs: 16 (grp1 - grp0) columns of each token
+    const int n0 = 16 * grp0, nc = min(width, N - n0);
+    for (int i = t; i < M * width; i += kThreads) {
+      const int m = i / width, c = i - m * width;
+      if (c < nc) a.out[(size_t)m * N + n0 + c] = outs[i];
+    }
+  } else {
+    zero_tail(xf);
+    zero_tail(wa);
+    products(wa, 0);
+    if constexpr (kTwo) {
+      zero_tail(wb);
+      products(wb, 1);
+    }
+    moe::lds_barrier();
+    if (!task) return;
+    if constexpr (EPI == kBiasResidual) {
+      const int n = w_row<EPI>(tgrp, 4 * g + ei);
+      const float tb = bf2f(f2bf(bf2f(f2bf(total(0, ei))) + bf2f(eb0)));
+      if (n < N) a.out[(size_t)tm * N + n] = f2bf(bf2f(er) + tb);
+    } else {
+      // bias (its own bf16 rounding), then YaRN RoPE of q / k heads exactly as
+      // the standalone append kernel does, then q out or the cache slot
+      const int head = erow / kD, d = erow % kD;  // dimensions d and d + 32
+      float lo = bf2f(f2bf(bf2f(f2bf(total(tgrp - grp0, ei))) + bf2f(eb0)));
+      float hi = bf2f(f2bf(bf2f(f2bf(total(tgrp - grp0, ei + 2))) + bf2f(eb1)));
+      if (head < kHq + kHkv) {
+        const float nl = lo * cs - hi * sn;
+        const float nh = lo * sn + hi * cs;
+        lo = nl;
+        hi = nh;
+      }
+      uint16_t* dst = nullptr;
+      if (head < kHq) {
+        dst = a.q_out + ((size_t)tm * kHq + head) * kD;
+      } else if (eslot >= 0 && eslot < a.num_pages * kPage) {  // other slots are not written
+        const int kv = head < kHq + kHkv ? 0 : 1;
+        const int hk = head - kHq - kv * kHkv;
+        dst = (uint16_t*)(a.cache + (size_t)(eslot / kPage) * kPageBytes +
+                          (size_t)(kv * kHkv + hk) * kHeadBlock + (eslot % kPage) * (kD * 2));
+      }
+      if (dst) {
+        dst[d] = f2bf(lo);
+        dst[d + 32] = f2bf(hi);
+      }
+    }
+  }
+}
+
+template <int EPI, bool kNorm>
+int launch(const Args& a, dim3 grid, size_t lds, hipStream_t s) {
+  const bool small = a.K <= 32 * 6 * kWaves;  // 6 steps a wave; 8 cover K <= 4096
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), lds, s, a);
+    return hipGetLastError() == hipSuccess ? 0 : -6;
+  };
+  return small ? go(rows_kernel<6, EPI, kNorm>) : go(rows_kernel<8, EPI, kNorm>);
+}
+
+}  // namespace rows
+
+extern "C" {
+
+// out = bf16(t W^T) for M <= 16 rows, t = x or RMSNorm(x)
+int attn_launch_rows_plain(const void* x, int M, int K, const void* W, int N, const void* norm_w,
+                           float eps, void* out, hipStream_t s) {
+  using namespace rows;
+  Args a{};
+  a.x = (const uint16_t*)x;
+  a.M = M;
+  a.K = K;
+  a.W = (const uint16_t*)W;
+  a.N = N;
+  a.norm_w = (const uint16_t*)norm_w;
+  a.eps = eps;
+  a.out = (uint16_t*)out;
+  const int64_t groups = ((int64_t)N + 15) / 16;
+  // one workgroup per CU, more where a range would be longer than kMaxGroups
+  const int64_t fill = groups < 256 ? groups : 256;
+  const int64_t need = (groups + kMaxGroups - 1) / kMaxGroups;
+  const dim3 grid((unsigned)(need > fill ? need : fill));
+  const int64_t range = (groups + grid.x - 1) / grid.x;
+  const size_t lds = (size_t)M * range * 16 * 2;
+  return norm_w ? launch<kPlain, true>(a, grid, lds, s) : launch<kPlain, false>(a, grid, lds, s);
+}
+
+// out = bf16(res + bf16(bf16(x W^T) + bias)), M <= 16
+int attn_launch_rows_bias_residual(const void* x, int M, int K, const void* W, int N,
+                                   const void* bias, const void* res, void* out, hipStream_t s) {
+  using namespace rows;
+  Args a{};
+  a.x = (const uint16_t*)x;
+  a.M = M;
+  a.K = K;
+  a.W = (const uint16_t*)W;
+  a.N = N;
+  a.out = (uint16_t*)out;
+  a.bias = (const uint16_t*)bias;
+  a.res = (const uint16_t*)res;
+  return launch<kBiasResidual, false>(a, dim3((unsigned)(((int64_t)N + 15) / 16)), 0, s);
+}
+
+// the QKV projection with bias, RoPE and the cache append, M <= 16
+int attn_launch_rows_qkv(const void* x, int M, int K, const void* W, const void* norm_w, float eps,
+                         const void* bias, const int* positions, const int* slots,
+                         const float* inv_freq, float conc, void* cache, int num_pages,
+                         void* q_out, hipStream_t s) {
+  using namespace rows;
+  Args a{};
+  a.x = (const uint16_t*)x;
+  a.M = M;
+  a.K = K;
+  a.W = (const uint16_t*)W;
+  a.N = (kHq + 2 * kHkv) * kD;
+  a.norm_w = (const uint16_t*)norm_w;
+  a.eps = eps;
+  a.bias = (const uint16_t*)bias;
+  a.positions = positions;
+  a.slots = slots;
+  a.inv_freq = inv_freq;
+  a.conc = conc;
+  a.cache = (uint8_t*)cache;
+  a.num_pages = num_pages;
+  a.q_out = (uint16_t*)q_out;
+  const dim3 grid(a.N / 32);
+  return norm_w ? launch<kQkv, true>(a, grid, 0, s) : launch<kQkv, false>(a, grid, 0, s);
+}
+
+}  // extern "C"

@@ -172,6 +172,42 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
+// sin and cos of a RoPE angle in fp64, within about 1e-16 (|a| < 2^50): the
+// angle less n pi/2 in two fused steps (pi/2 as the nearest double and the
+// nearest double of the rest, Cody and Waite), then both Taylor series on
+// [-pi/4, pi/4] (to y^15 and y^16: the first terms left out are below 5e-17)
+// and the quadrant.  About 30 instructions and a few registers, where the
+// library's pair carries the reduction for arguments of any size: it spilled
+// in kernels that hold their weights in flight, and the prefill epilogue was
+// bound by it (4096 tokens: 52 us).
+__device__ __forceinline__ void sincos_f64(double a, double& s, double& c) {
+  const double n = __builtin_rint(a * 0x1.45f306dc9c883p-1);
+  double y = __builtin_fma(-n, 0x1.921fb54442d18p+0, a);
+  y = __builtin_fma(-n, 0x1.1a62633145c07p-54, y);
+  const double z = y * y;
+  double ps = -1.0 / 1307674368000.0, pc = 1.0 / 20922789888000.0;
+  ps = __builtin_fma(ps, z, 1.0 / 6227020800.0);
+  ps = __builtin_fma(ps, z, -1.0 / 39916800.0);
+  ps = __builtin_fma(ps, z, 1.0 / 362880.0);
+  ps = __builtin_fma(ps, z, -1.0 / 5040.0);
+  ps = __builtin_fma(ps, z, 1.0 / 120.0);
+  ps = __builtin_fma(ps, z, -1.0 / 6.0);
+  ps = __builtin_fma(ps, z, 1.0);
+  pc = __builtin_fma(pc, z, -1.0 / 87178291200.0);
+  pc = __builtin_fma(pc, z, 1.0 / 479001600.0);
+  pc = __builtin_fma(pc, z, -1.0 / 3628800.0);
+  pc = __builtin_fma(pc, z, 1.0 / 40320.0);
+  pc = __builtin_fma(pc, z, -1.0 / 720.0);
+  pc = __builtin_fma(pc, z, 1.0 / 24.0);
+  pc = __builtin_fma(pc, z, -0.5);
+  pc = __builtin_fma(pc, z, 1.0);
+  ps *= y;
+  const int q = (int)(n - 4.0 * __builtin_floor(n * 0.25));  // quadrant 0..3
+  const double u = (q & 1) ? pc : ps, v = (q & 1) ? ps : pc;
+  s = (q & 2) ? -u : u;
+  c = ((q + 1) & 2) ? -v : v;
+}
+
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
 #pragma unroll

@@ -7,8 +7,8 @@
  * q and k, append_mha_kv, self_attention (prefill) / cross_attention (decode)
  * / both merged (extend), the sink scaling, the output nn.Linear and the
  * residual add.  The dense projections (QKV, output, unembedding) are
- * library GEMMs on the host side for prefill-sized inputs and the GEMV entry
- * points below (with their epilogues fused) for decode-sized ones.
+ * library GEMMs on the host side for prefill-sized inputs and the GEMV and
+ * rows entry points below (with their epilogues fused) for decode-sized ones.
  * The conventions of moe_gfx950.h hold: caller-owned device buffers, nothing
  * allocated, no host synchronisation, the stream last, MOE_OK or a negative
  * MOE_ERR_* code (no launch on error).
@@ -118,6 +118,17 @@ MOE_API int attn_gemv_bias_residual(const uint16_t* x, int64_t M, int64_t K, con
  * W [5120, K], then the bias, YaRN RoPE, q_out and the cache append exactly
  * as attn_qkv_rope_append does. */
 MOE_API int attn_qkv_gemv_rope_append(const uint16_t* x, int64_t M, int64_t K, const uint16_t* W,
+                                      const uint16_t* norm_w, float eps,
+                                      const uint16_t* qkv_bias, const int32_t* positions,
+                                      const int32_t* slots, const float* inv_freq,
+                                      float concentration, void* kv_cache, int64_t num_pages,
+                                      uint16_t* q_out, moe_stream_t stream);
+
+/* The same two projections for decode batches of up to 16 tokens. */
+MOE_API int attn_rows_bias_residual(const uint16_t* x, int64_t M, int64_t K, const uint16_t* W,
+                                    int64_t N, const uint16_t* bias, const uint16_t* residual,
+                                    uint16_t* out, moe_stream_t stream);
+MOE_API int attn_rows_qkv_rope_append(const uint16_t* x, int64_t M, int64_t K, const uint16_t* W,
                                       const uint16_t* norm_w, float eps,
                                       const uint16_t* qkv_bias, const int32_t* positions,
                                       const int32_t* slots, const float* inv_freq,

@@ -382,3 +382,71 @@ def test_gemv_kernels(A, M):
         pg, sl = divmod(int(slots[i]), PAGE)
         _ulp_close(c[pg, 0, :, sl], rk[i], "k", frac=0.03)
         _ulp_close(c[pg, 1, :, sl], rv[i], "v", frac=0.03)
+
+
+@pytest.mark.parametrize("M,K,N", [(2, 8, 1), (3, 40, 17), (5, 2888, 31), (8, 3080, 100),
+                                   (7, 64, 12309), (2, 16, 270001), (8, 4096, 528)])
+def test_gemv_several_tokens_edges(A, M, K, N):
+    """Two to eight tokens at the edges of the matrix-core form: K below, at and
+    past whole 32-wide steps and both register sizes, one row group, ranges of
+    two and three groups with a ragged last one, more groups than the
+    workgroups' ranges hold.  The sums differ from the oracle's fp64 by fp32
+    rounding only, so a result off by more than one bf16 ulp is wrong."""
+    rng = np.random.default_rng(K + N)
+    x = bf(np.abs(rng.standard_normal((M, K))) + 0.1)
+    W = bf(rng.standard_normal((N, K)) * 0.02)
+    _ulp_close(host_bf16(A.gemv(bf16_dev(x), bf16_dev(W))), AO.linear(x, W, None), "gemv")
+    nw = bf(rng.uniform(0.5, 1.5, K))
+    got = host_bf16(A.gemv(bf16_dev(x), bf16_dev(W), norm_w=bf16_dev(nw), eps=1e-5))
+    _ulp_close(got, AO.linear(O.rms_norm(x, nw, 1e-5), W, None), "norm + gemv")
+    # what lies past a row's end or past the last row enters no sum
+    W[-1, -1] = bf(np.array([np.inf]))[0]
+    y = O.bf16_to_f32(host_bf16(A.gemv(bf16_dev(x), bf16_dev(W))))
+    assert np.isinf(y[:, -1]).all() and np.isfinite(y[:, :-1]).all()
+
+
+def _rope_close(got, ref, what):
+    """As _ulp_close, for rotated pairs (d, d + 32): a projection one bf16 ulp
+    off moves both results of its pair by up to an ulp of the pair's length,
+    times the concentration (1.35) and sqrt(2) for both inputs, and the final
+    rounding adds one: at most 3 ulps of the length."""
+    g, r = O.bf16_to_f32(got).astype(np.float64), O.bf16_to_f32(ref).astype(np.float64)
+    length = np.hypot(r[..., :D // 2], r[..., D // 2:]).astype(np.float32)
+    bound = 3 * np.spacing(np.concatenate([length, length], -1)).astype(np.float64) * 2 ** 16
+    diff = np.abs(g - r)
+    assert (diff > 0).mean() <= 0.03 and np.all(diff <= bound), (what, (diff / bound).max())
+
+
+@pytest.mark.parametrize("M", [9, 16])
+def test_rows_projections(A, M):
+    """The two layer projections at 9 and 16 tokens, against the oracle."""
+    rng = np.random.default_rng(70 + M)
+    K = 2880
+    x = O.make_input(71, M)
+    nw = bf(rng.uniform(0.5, 1.5, K))
+    W = bf(rng.standard_normal((A.QKV_DIM, K)) * 0.02)
+    b = bf(rng.standard_normal(A.QKV_DIM) * 0.01)
+    pos = (np.arange(M, dtype=np.int32) * 9999) % 131072
+    slots = rng.choice(4 * PAGE, M, replace=False).astype(np.int32)
+    slots[1] = 4 * PAGE                                # outside the pool: not written
+    cache = torch.zeros((4, 2, HKV, PAGE, D), dtype=torch.bfloat16, device="cuda")
+    q = torch.empty((M, HQ, D), dtype=torch.bfloat16, device="cuda")
+    inv, conc = _inv_freq_dev()
+    A.rows_qkv_rope_append(bf16_dev(x), bf16_dev(W), bf16_dev(b), i32_dev(pos), i32_dev(slots),
+                           inv, conc, cache, q, norm_w=bf16_dev(nw))
+    rq, rk, rv = AO.split_qkv(AO.linear(O.rms_norm(x, nw, 1e-5), W, b))
+    _rope_close(host_bf16(q), AO.rope(rq, pos), "q")
+    rk, c = AO.rope(rk, pos), host_bf16(cache)
+    for i in range(M):
+        if slots[i] < 4 * PAGE:
+            pg, sl = divmod(int(slots[i]), PAGE)
+            _rope_close(c[pg, 0, :, sl], rk[i], "k")
+            _ulp_close(c[pg, 1, :, sl], rv[i], "v", frac=0.03)
+            c[pg, :, :, sl] = 0
+    assert not c.any()
+    o = bf(rng.standard_normal((M, 4096)) * 0.3)
+    Wo = bf(rng.standard_normal((K + 7, 4096)) * 0.02)
+    y = AO.linear(o, Wo, None)
+    zero, res = bf(np.zeros(K + 7)), bf(np.zeros((M, K + 7)))
+    got = host_bf16(A.rows_bias_residual(bf16_dev(o), bf16_dev(Wo), bf16_dev(zero), bf16_dev(res)))
+    _ulp_close(got, y, "out projection")
