@@ -57,26 +57,72 @@ struct PageList {
 // ---------------------------------------------------------------------------
 // RMSNorm (attention.py:80, nn.RMSNorm): sum of squares of the bf16 inputs in
 // fp64 (exact for inputs spanning less than 2^37), r = fp32(1/sqrt(ss/H +
-// eps)) in fp64, t = bf16(fp32(x r) w).  One 256-thread workgroup per token.
-__global__ __launch_bounds__(256) void rms_norm_kernel(const uint16_t* __restrict__ x, int H,
-                                                       const uint16_t* __restrict__ w, float eps,
-                                                       uint16_t* __restrict__ out) {
-  __shared__ double part[4];
-  const int tok = blockIdx.x;
-  const uint16_t* xr = x + (size_t)tok * H;
+// eps)) in fp64, t = bf16(fp32(x r) w).  One workgroup of three waves per token,
+// 16-byte loads; a row of up to 6144 (two rounds of loads at gpt-oss's 2880)
+// stays in registers between the two passes, all of its loads and the norm
+// weight's in flight at once.  Bound by the row's bytes where there are many
+// tokens, by one memory round trip where there are few (one pass each of
+// 2-byte loads in 256 threads before: 4096 tokens 18.0 -> 9.5 us, 64 tokens 4.2 ->
+// 2.4).
+constexpr int kRmsThreads = 192;
+constexpr int kRmsHeld = 4;  // 16-byte chunks of a row that a thread holds
+
+__device__ __forceinline__ double rms_sq(u32x4 v) {
   double ss = 0.0;
-  for (int i = threadIdx.x; i < H; i += 256) {
-    const double v = (double)bf2f(xr[i]);
-    ss += v * v;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const double lo = (double)__uint_as_float(v[j] << 16);
+    const double hi = (double)__uint_as_float(v[j] & 0xFFFF0000u);
+    ss += lo * lo + hi * hi;
+  }
+  return ss;
+}
+
+__device__ __forceinline__ u32x4 rms_scale(u32x4 v, u32x4 w, float r) {
+  u32x4 o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t lo = f2bf(__fmul_rn(__fmul_rn(__uint_as_float(v[j] << 16), r),
+                                       __uint_as_float(w[j] << 16)));
+    const uint32_t hi = f2bf(__fmul_rn(__fmul_rn(__uint_as_float(v[j] & 0xFFFF0000u), r),
+                                       __uint_as_float(w[j] & 0xFFFF0000u)));
+    o[j] = lo | (hi << 16);
+  }
+  return o;
+}
+
+template <int kChunks>  // chunks a thread holds; 0: the row is read twice
+__global__ __launch_bounds__(kRmsThreads) void rms_norm_kernel(const u32x4* __restrict__ x, int H,
+                                                               const u32x4* __restrict__ w,
+                                                               float eps,
+                                                               u32x4* __restrict__ out) {
+  __shared__ double part[kRmsThreads / kWave];
+  const int chunks = H / 8, t = threadIdx.x;
+  const size_t row = (size_t)blockIdx.x * chunks;
+  u32x4 v[kChunks + 1], wv[kChunks + 1];
+  double ss = 0.0;
+  if constexpr (kChunks > 0) {
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i) v[i] = x[row + min(t + i * kRmsThreads, chunks - 1)];
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i) wv[i] = w[min(t + i * kRmsThreads, chunks - 1)];
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i) ss += t + i * kRmsThreads < chunks ? rms_sq(v[i]) : 0.0;
+  } else {
+    for (int c = t; c < chunks; c += kRmsThreads) ss += rms_sq(x[row + c]);
   }
   ss = moe::wave_sum(ss);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
-  __syncthreads();
-  const double tot = (part[0] + part[1]) + (part[2] + part[3]);
+  if ((t & 63) == 0) part[t >> 6] = ss;
+  moe::lds_barrier();
+  const double tot = (part[0] + part[1]) + part[2];
   const float r = (float)(1.0 / sqrt(tot / (double)H + (double)eps));
-  for (int i = threadIdx.x; i < H; i += 256) {
-    const float xv = __fmul_rn(bf2f(xr[i]), r);
-    out[(size_t)tok * H + i] = f2bf(__fmul_rn(xv, bf2f(w[i])));
+  if constexpr (kChunks > 0) {
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i)
+      if (t + i * kRmsThreads < chunks)
+        out[row + t + i * kRmsThreads] = rms_scale(v[i], wv[i], r);
+  } else {
+    for (int c = t; c < chunks; c += kRmsThreads) out[row + c] = rms_scale(x[row + c], w[c], r);
   }
 }
 
@@ -87,42 +133,83 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const uint16_t* __restric
 // cos/sin of fp32(position) * inv_freq are evaluated in fp64, rounded to fp32
 // and then to bf16 (the rope's .astype(dtype)), then scaled by the fp32
 // concentration; the rotation rounds each product and the difference / sum
-// separately (no contraction).  One thread per rotation pair (d, d + 32):
-// 256 threads = 8 heads of one token; grid (10, n).
-__global__ __launch_bounds__(256) void qkv_rope_append_kernel(
-    const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ bias,
+// separately (no contraction).  A workgroup takes kRopeTok tokens; their 32
+// cos/sin pairs each are taken once, for all 72 heads, into LDS (one pair per
+// thread and (head, d) before: bound by the fp64 sine and cosine, 52 us at
+// 4096 tokens against 14.6 now, 5.8 TB/s of its 84 MB in and out), while
+// the first token's loads are in flight.  One thread per eight rotation pairs
+// (d .. d + 7, + 32) of a head: 16-byte loads and stores.
+constexpr int kRopeThreads = kQkvHeads * 4;  // 320: (head, quarter of its 32 pairs)
+
+template <int kRopeTok>
+__global__ __launch_bounds__(kRopeThreads) void qkv_rope_append_kernel(
+    const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ bias, int n,
     const int* __restrict__ positions, const int* __restrict__ slots,
     const float* __restrict__ inv_freq, float conc, uint8_t* __restrict__ cache, int num_pages,
     uint16_t* __restrict__ q_out) {
 #pragma clang fp contract(off)
-  const int tok = blockIdx.y;
-  const int head = blockIdx.x * 8 + (threadIdx.x >> 5);
-  const int d = threadIdx.x & 31;
-  const size_t base = (size_t)tok * (kQkvHeads * kD) + head * kD;
-  float lo = bf2f(f2bf(bf2f(qkv[base + d]) + bf2f(bias[head * kD + d])));
-  float hi = bf2f(f2bf(bf2f(qkv[base + d + 32]) + bf2f(bias[head * kD + d + 32])));
-  const int slot = slots[tok];
-  if (head < kHq + kHkv) {
-    const float freq = (float)positions[tok] * inv_freq[d];
-    const double fd = (double)freq;
-    const float c = bf2f(f2bf((float)cos(fd))) * conc;
-    const float s = bf2f(f2bf((float)sin(fd))) * conc;
-    const float nlo = lo * c - hi * s;
-    const float nhi = lo * s + hi * c;
-    lo = nlo;
-    hi = nhi;
+  __shared__ float cs[kRopeTok][32], sn[kRopeTok][32];
+  const int t = threadIdx.x;
+  const int tok0 = blockIdx.x * kRopeTok, ntok = min(kRopeTok, n - tok0);
+  const int head = t >> 2, d = (t & 3) * 8;
+  const size_t col = (size_t)head * kD + d;
+  u32x4 lo[kRopeTok], hi[kRopeTok];
+  int slot[kRopeTok];
+#pragma unroll
+  for (int j = 0; j < kRopeTok; ++j) {
+    const int tok = tok0 + min(j, ntok - 1);
+    const uint16_t* src = qkv + (size_t)tok * (kQkvHeads * kD) + col;
+    lo[j] = *(const u32x4*)src;
+    hi[j] = *(const u32x4*)(src + 32);
+    slot[j] = slots[tok];
   }
-  const uint16_t blo = f2bf(lo), bhi = f2bf(hi);
-  if (head < kHq) {
-    uint16_t* qo = q_out + ((size_t)tok * kHq + head) * kD;
-    qo[d] = blo;
-    qo[d + 32] = bhi;
-  } else if (slot >= 0 && slot < num_pages * kPage) {  // other slots are not written
-    const int kv = head < kHq + kHkv ? 0 : 1;
-    const int hk = head - kHq - kv * kHkv;
-    uint16_t* row = (uint16_t*)kv_row(cache, slot / kPage, kv, hk, slot % kPage);
-    row[d] = blo;
-    row[d + 32] = bhi;
+  const u32x4 blo = *(const u32x4*)(bias + col), bhi = *(const u32x4*)(bias + col + 32);
+  if (t < 32 * kRopeTok) {
+    const int j = t >> 5;
+    const float freq = (float)positions[tok0 + min(j, ntok - 1)] * inv_freq[t & 31];
+    double s, c;
+    moe::sincos_f64((double)freq, s, c);
+    cs[j][t & 31] = bf2f(moe::f64_to_bf16_via_f32(c)) * conc;
+    sn[j][t & 31] = bf2f(moe::f64_to_bf16_via_f32(s)) * conc;
+  }
+  moe::lds_barrier();
+#pragma unroll
+  for (int j = 0; j < kRopeTok; ++j) {
+    if (j >= ntok) break;
+    u32x4 olo, ohi;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t wl = 0, wh = 0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {  // the word's two dimensions
+        auto val = [&](uint32_t w) { return __uint_as_float(h ? w & 0xFFFF0000u : w << 16); };
+        float l = bf2f(f2bf(val(lo[j][i]) + val(blo[i])));
+        float u = bf2f(f2bf(val(hi[j][i]) + val(bhi[i])));
+        if (head < kHq + kHkv) {
+          const float c = cs[j][d + 2 * i + h], s = sn[j][d + 2 * i + h];
+          const float nl = l * c - u * s;
+          const float nu = l * s + u * c;
+          l = nl;
+          u = nu;
+        }
+        wl |= (uint32_t)f2bf(l) << (16 * h);
+        wh |= (uint32_t)f2bf(u) << (16 * h);
+      }
+      olo[i] = wl;
+      ohi[i] = wh;
+    }
+    uint16_t* dst = nullptr;
+    if (head < kHq) {
+      dst = q_out + ((size_t)(tok0 + j) * kHq + head) * kD;
+    } else if (slot[j] >= 0 && slot[j] < num_pages * kPage) {  // other slots are not written
+      const int kv = head < kHq + kHkv ? 0 : 1;
+      const int hk = head - kHq - kv * kHkv;
+      dst = (uint16_t*)kv_row(cache, slot[j] / kPage, kv, hk, slot[j] % kPage);
+    }
+    if (dst) {
+      *(u32x4*)(dst + d) = olo;
+      *(u32x4*)(dst + d + 32) = ohi;
+    }
   }
 }
 
@@ -838,18 +925,29 @@ extern "C" {
 
 int attn_launch_rms_norm(const void* x, int n, int H, const void* w, float eps, void* out,
                          hipStream_t s) {
-  hipLaunchKernelGGL(attn::rms_norm_kernel, dim3(n), dim3(256), 0, s, (const uint16_t*)x, H,
-                     (const uint16_t*)w, eps, (uint16_t*)out);
-  return hipGetLastError() == hipSuccess ? 0 : -6;
+  using namespace attn;
+  // gpt-oss's row fits two chunks a thread; longer ones are held up to kRmsHeld
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(n), dim3(kRmsThreads), 0, s, (const u32x4*)x, H,
+                       (const u32x4*)w, eps, (u32x4*)out);
+    return hipGetLastError() == hipSuccess ? 0 : -6;
+  };
+  if (H <= 8 * kRmsThreads * 2) return go(rms_norm_kernel<2>);
+  return H <= 8 * kRmsThreads * kRmsHeld ? go(rms_norm_kernel<kRmsHeld>) : go(rms_norm_kernel<0>);
 }
 
 int attn_launch_qkv_rope_append(const void* qkv, const void* bias, int n, const int* positions,
                                 const int* slots, const float* inv_freq, float conc, void* cache,
                                 int num_pages, void* q_out, hipStream_t s) {
-  hipLaunchKernelGGL(attn::qkv_rope_append_kernel, dim3(attn::kQkvHeads / 8, n), dim3(256), 0, s,
-                     (const uint16_t*)qkv, (const uint16_t*)bias, positions, slots, inv_freq, conc,
-                     (uint8_t*)cache, num_pages, (uint16_t*)q_out);
-  return hipGetLastError() == hipSuccess ? 0 : -6;
+  // several tokens a workgroup once there are workgroups enough without
+  auto go = [&](auto kernel, int per) {
+    hipLaunchKernelGGL(kernel, dim3((n + per - 1) / per), dim3(attn::kRopeThreads), 0, s,
+                       (const uint16_t*)qkv, (const uint16_t*)bias, n, positions, slots, inv_freq,
+                       conc, (uint8_t*)cache, num_pages, (uint16_t*)q_out);
+    return hipGetLastError() == hipSuccess ? 0 : -6;
+  };
+  return n >= 4096 ? go(attn::qkv_rope_append_kernel<4>, 4)
+                   : go(attn::qkv_rope_append_kernel<1>, 1);
 }
 
 int attn_launch_decode(const void* q, int batch, const void* cache, const int* page_indptr,

@@ -450,3 +450,34 @@ def test_rows_projections(A, M):
     zero, res = bf(np.zeros(K + 7)), bf(np.zeros((M, K + 7)))
     got = host_bf16(A.rows_bias_residual(bf16_dev(o), bf16_dev(Wo), bf16_dev(zero), bf16_dev(res)))
     _ulp_close(got, y, "out projection")
+
+
+@pytest.mark.parametrize("n,H", [(1, 8), (3, 2880), (2, 3072), (2, 3080), (2, 6144), (2, 6152)])
+def test_rms_norm_row_sizes(A, n, H):
+    """Rows held in registers at both sizes, and read twice, bit for bit."""
+    rng = np.random.default_rng(H)
+    x, w = bf(rng.standard_normal((n, H))), bf(rng.uniform(0.5, 1.5, H))
+    np.testing.assert_array_equal(host_bf16(A.rms_norm(bf16_dev(x), bf16_dev(w), 1e-5)),
+                                  O.rms_norm(x, w, 1e-5))
+
+
+@pytest.mark.parametrize("n", [4096, 4099])
+def test_qkv_rope_append_many_tokens(A, n):
+    """Four tokens a workgroup, with and without a ragged last one, at positions
+    over the whole context, bit for bit."""
+    rng = np.random.default_rng(n)
+    qkv = bf(rng.standard_normal((n, A.QKV_DIM)))
+    bias = bf(rng.standard_normal(A.QKV_DIM) * 0.1)
+    pos = rng.integers(0, 131072, n).astype(np.int32)
+    pages = -(-n // PAGE)
+    slots = rng.permutation(n).astype(np.int32)
+    cache = torch.zeros((pages, 2, HKV, PAGE, D), dtype=torch.bfloat16, device="cuda")
+    q = torch.empty((n, HQ, D), dtype=torch.bfloat16, device="cuda")
+    inv, conc = _inv_freq_dev()
+    A.qkv_rope_append(bf16_dev(qkv), bf16_dev(bias), i32_dev(pos), i32_dev(slots), inv, conc,
+                      cache, q)
+    rq, rk, rv = AO.split_qkv(AO.bias_add(qkv, bias))
+    np.testing.assert_array_equal(host_bf16(q), AO.rope(rq, pos))
+    c = host_bf16(cache).transpose(0, 3, 1, 2, 4).reshape(-1, 2, HKV, D)
+    np.testing.assert_array_equal(c[slots, 0], AO.rope(rk, pos))
+    np.testing.assert_array_equal(c[slots, 1], rv)
