@@ -29,6 +29,9 @@ _SIGS = {
     "attn_decode_workspace_bytes": ([_I64, _I64], _SZ),
     "attn_decode": ([_P, _I64, _P, _I64, _P, _P, _P, _I64, _I32, _F, _P, _P, _P, _SZ, _P], _INT),
     "attn_prefill": ([_P, _P, _I64, _I64, _P, _I64, _P, _P, _P, _I32, _F, _P, _P, _P], _INT),
+    "attn_prefill_workspace_bytes": ([_I64, _I64, _I64, _I64, _I32], _SZ),
+    "attn_prefill_split": ([_P, _I64, _P, _I64, _I64, _P, _I64, _P, _P, _P, _I64, _I32, _F, _P, _P,
+                            _P, _SZ, _P], _INT),
     "attn_bias_residual": ([_P, _P, _P, _I64, _I64, _P, _P], _INT),
     "attn_embedding": ([_P, _I64, _P, _I64, _I64, _P, _P], _INT),
     "attn_gemv": ([_P, _I64, _I64, _P, _I64, _P, _F, _P, _P], _INT),
@@ -129,8 +132,13 @@ def decode(q: torch.Tensor, kv_cache: torch.Tensor, page_indptr: torch.Tensor,
 
 def prefill(q: torch.Tensor, q_indptr: torch.Tensor, max_q_len: int, kv_cache: torch.Tensor,
             page_indptr: torch.Tensor, page_indices: torch.Tensor, kv_len: torch.Tensor,
-            window: int, sm_scale: float, sinks: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
-    """Causal (sliding-window) attention of each sequence's new tokens over its cache."""
+            window: int, sm_scale: float, sinks: torch.Tensor, out: torch.Tensor,
+            max_kv_len: int = 0) -> torch.Tensor:
+    """Causal (sliding-window) attention of each sequence's new tokens over its cache.
+
+    ``max_kv_len`` (0: unknown) bounds kv_len; with it, calls of few query tiles
+    over many keys share the keys out over more workgroups (their partial
+    results in a buffer allocated for the call)."""
     _expect(q, "q", torch.bfloat16)
     n = q.shape[0]
     _expect(q, "q", torch.bfloat16, (n, Q_HEADS, HEAD_DIM))
@@ -139,6 +147,15 @@ def prefill(q: torch.Tensor, q_indptr: torch.Tensor, max_q_len: int, kv_cache: t
     _tables(kv_cache, page_indptr, page_indices, kv_len, batch)
     _expect(sinks, "sinks", torch.bfloat16, (Q_HEADS,))
     _expect(out, "out", torch.bfloat16, (n, Q_HEADS, HEAD_DIM))
+    need = _lib.attn_prefill_workspace_bytes(n, batch, max_q_len, max_kv_len, window)
+    if need:
+        ws = torch.empty(need, dtype=torch.uint8, device=q.device)
+        _check(_lib.attn_prefill_split(_ptr(q), n, _ptr(q_indptr), batch, max_q_len,
+                                       _ptr(kv_cache), kv_cache.shape[0], _ptr(page_indptr),
+                                       _ptr(page_indices), _ptr(kv_len), max_kv_len, window,
+                                       sm_scale, _ptr(sinks), _ptr(out), _ptr(ws), need,
+                                       _stream()), "attn_prefill_split")
+        return out
     _check(_lib.attn_prefill(_ptr(q), _ptr(q_indptr), batch, max_q_len, _ptr(kv_cache),
                              kv_cache.shape[0], _ptr(page_indptr), _ptr(page_indices),
                              _ptr(kv_len), window, sm_scale, _ptr(sinks), _ptr(out), _stream()),

@@ -5,6 +5,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "../../include/attn_gfx950.h"
 
 extern "C" {
@@ -20,7 +22,8 @@ int attn_launch_decode(const void* q, int batch, const void* cache, const int* p
 int attn_launch_prefill(const void* q, const int* q_indptr, int batch, int max_q_len,
                         const void* cache, const int* page_indptr, const int* page_indices,
                         int num_pages, const int* kv_len, int window, float sm_scale,
-                        const void* sinks, void* out, hipStream_t s);
+                        const void* sinks, void* out, int splits, int rows, float* part_o,
+                        float* part_ml, hipStream_t s);
 int attn_launch_bias_residual(const void* x, const void* y, const void* bias, int64_t n, int H,
                               void* out, hipStream_t s);
 int attn_launch_embedding(const int* ids, int n, const void* table, int vocab, int H, void* out,
@@ -68,6 +71,22 @@ int64_t decode_cps(int64_t batch) { return batch >= 32 ? 8 : batch >= 8 ? 4 : ba
 int64_t decode_splits(int64_t batch, int64_t max_span) {
   const int64_t keys = kDecChunk * decode_cps(batch);
   return (max_span + keys - 1) / keys;
+}
+
+// Workgroups that a tile's keys are shared out over in prefill attention: as many
+// as fit the chip at once (a tile has 16 workgroups, a CU holds two), each with
+// about 192 keys or more (a causal tile sees half of the new ones), at most 16.
+// Measured, us without and with (new tokens + cached): 9 + 1500 60.6 and 18.3, 64 +
+// 8000 296 and 37.7, 300 + 600 43.3 and 31.4, 300 + 6000 238 and 86, 1024 + 0 46.3 and
+// 45.2.  One round more than fits cost more than the shares gained (300 + 6000 in
+// 560 workgroups 104 us); 700 + 0 in two shares took 35.3 against 33.3.
+constexpr int64_t kPfSplitKeys = 192, kPfMaxSplits = 16, kPfWorkgroups = 512;
+int64_t prefill_splits(int64_t batch, int64_t max_q_len, int64_t max_kv_len, int64_t window) {
+  const int64_t wgs = (max_q_len + 63) / 64 * batch * 16;
+  const int64_t keys = (window > 0 ? std::min(max_kv_len, window + 64) : max_kv_len) - max_q_len / 2;
+  if (wgs <= 0) return 1;
+  const int64_t s = std::min(kPfWorkgroups / wgs, keys / kPfSplitKeys);
+  return std::max<int64_t>(1, std::min(s, kPfMaxSplits));
 }
 
 }  // namespace
@@ -136,10 +155,11 @@ int attn_decode(const uint16_t* q, int64_t batch, const void* kv_cache, int64_t 
                                    as_stream(stream)));
 }
 
-int attn_prefill(const uint16_t* q, const int32_t* q_indptr, int64_t batch, int64_t max_q_len,
-                 const void* kv_cache, int64_t num_pages, const int32_t* page_indptr,
-                 const int32_t* page_indices, const int32_t* kv_len, int32_t window,
-                 float sm_scale, const uint16_t* sinks, uint16_t* out, moe_stream_t stream) {
+static int prefill(const uint16_t* q, int64_t rows, const int32_t* q_indptr, int64_t batch,
+                   int64_t max_q_len, const void* kv_cache, int64_t num_pages,
+                   const int32_t* page_indptr, const int32_t* page_indices, const int32_t* kv_len,
+                   int64_t splits, int32_t window, float sm_scale, const uint16_t* sinks,
+                   uint16_t* out, float* part_o, float* part_ml, moe_stream_t stream) {
   if (batch < 0 || max_q_len < 0 || max_q_len > kMaxTokens || num_pages <= 0 ||
       num_pages > kMaxPages)
     return MOE_ERR_SHAPE;
@@ -153,7 +173,46 @@ int attn_prefill(const uint16_t* q, const int32_t* q_indptr, int64_t batch, int6
     return MOE_ERR_ALIGN;
   return status(attn_launch_prefill(q, q_indptr, (int)batch, (int)max_q_len, kv_cache,
                                     page_indptr, page_indices, (int)num_pages, kv_len, window,
-                                    sm_scale, sinks, out, as_stream(stream)));
+                                    sm_scale, sinks, out, (int)splits, (int)rows, part_o, part_ml,
+                                    as_stream(stream)));
+}
+
+int attn_prefill(const uint16_t* q, const int32_t* q_indptr, int64_t batch, int64_t max_q_len,
+                 const void* kv_cache, int64_t num_pages, const int32_t* page_indptr,
+                 const int32_t* page_indices, const int32_t* kv_len, int32_t window,
+                 float sm_scale, const uint16_t* sinks, uint16_t* out, moe_stream_t stream) {
+  return prefill(q, 0, q_indptr, batch, max_q_len, kv_cache, num_pages, page_indptr, page_indices,
+                 kv_len, 1, window, sm_scale, sinks, out, nullptr, nullptr, stream);
+}
+
+// Workspace: the shares' o [splits][rows][64][64], then (m, l) [splits][rows][64][2]
+size_t attn_prefill_workspace_bytes(int64_t rows, int64_t batch, int64_t max_q_len,
+                                    int64_t max_kv_len, int32_t window) {
+  if (rows <= 0 || rows > kMaxTokens || batch <= 0 || max_q_len <= 0 || max_q_len > kMaxTokens)
+    return 0;
+  const int64_t splits = prefill_splits(batch, max_q_len, max_kv_len, window);
+  return splits <= 1 ? 0 : (size_t)(splits * rows * kQHeads * (kHeadDim + 2)) * sizeof(float);
+}
+
+int attn_prefill_split(const uint16_t* q, int64_t rows, const int32_t* q_indptr, int64_t batch,
+                       int64_t max_q_len, const void* kv_cache, int64_t num_pages,
+                       const int32_t* page_indptr, const int32_t* page_indices,
+                       const int32_t* kv_len, int64_t max_kv_len, int32_t window, float sm_scale,
+                       const uint16_t* sinks, uint16_t* out, void* workspace,
+                       size_t workspace_bytes, moe_stream_t stream) {
+  if (rows < 0 || rows > kMaxTokens) return MOE_ERR_SHAPE;
+  const size_t need = attn_prefill_workspace_bytes(rows, batch, max_q_len, max_kv_len, window);
+  if (need == 0)
+    return prefill(q, rows, q_indptr, batch, max_q_len, kv_cache, num_pages, page_indptr,
+                   page_indices, kv_len, 1, window, sm_scale, sinks, out, nullptr, nullptr, stream);
+  if (!workspace) return MOE_ERR_NULL;
+  if (!a16(workspace)) return MOE_ERR_ALIGN;
+  if (workspace_bytes < need) return MOE_ERR_WORKSPACE;
+  const int64_t splits = prefill_splits(batch, max_q_len, max_kv_len, window);
+  float* part_o = (float*)workspace;
+  return prefill(q, rows, q_indptr, batch, max_q_len, kv_cache, num_pages, page_indptr,
+                 page_indices, kv_len, splits, window, sm_scale, sinks, out, part_o,
+                 part_o + splits * rows * kQHeads * kHeadDim, stream);
 }
 
 int attn_bias_residual(const uint16_t* x, const uint16_t* y, const uint16_t* bias, int64_t n,

@@ -591,6 +591,11 @@ __device__ void decode_merge_group(const float* part_o, const float* part_ml, in
 //    read from a transposed LDS tile whose 32-key halves are interleaved
 //    (position 2i key i, 2i + 1 key i + 16), so that a lane's 8 keys are one
 //    16-byte read.
+//
+// kSplit: few query tiles over many keys (the next turn of a chat) leave most
+// CUs without a workgroup: each tile's key blocks are then shared out over
+// `splits` workgroups, which leave o (not normalised), the reference point m and
+// l of their share in the workspace for prefill_merge_kernel.
 constexpr int kPfQ = 64;              // query rows per wave
 constexpr int kPfSub = kPfQ / 16;     // 16-row subtiles per wave
 constexpr int kPfKeys = 64;           // keys per block
@@ -614,12 +619,14 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+template <bool kSplit>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void prefill_kernel(
     const uint16_t* __restrict__ q, const int* __restrict__ q_indptr,
     const uint8_t* __restrict__ cache, const int* __restrict__ page_indptr,
     const int* __restrict__ page_indices, int num_pages, const int* __restrict__ kv_len,
     int window, float sm_scale, const uint16_t* __restrict__ sinks, int tiles_per_seq,
-    uint16_t* __restrict__ out) {
+    uint16_t* __restrict__ out, int splits, int rows, float* __restrict__ part_o,
+    float* __restrict__ part_ml) {
   __shared__ __align__(16) uint16_t kt[2][kPfKeys * kKRow];
   __shared__ __align__(16) uint16_t vt[2][kD * kVRow];
   // each lane's Q operands, parked in LDS (a lane reads back only what it
@@ -635,7 +642,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   const int lin = (int)(blockIdx.x + blockIdx.y * gridDim.x);
   const int per_tile = (int)(gridDim.x / tiles_per_seq) * kPfHalves * kHkv;
   const int tile = tiles_per_seq - 1 - lin / per_tile;
-  const int rest = lin % per_tile;
+  const int share = kSplit ? lin % per_tile / (per_tile / splits) : 0;
+  const int rest = kSplit ? lin % (per_tile / splits) : lin % per_tile;
   const int b = rest / (kPfHalves * kHkv), half = rest / kHkv % kPfHalves, hk = rest % kHkv;
   const int qb = q_indptr[b], qn = q_indptr[b + 1] - qb;
   const int q0 = tile * kPfQ;
@@ -669,9 +677,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     for (int dt = 0; dt < 4; ++dt) o[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const int qlast = min(q0 + kPfQ, qn) - 1;
-  const int kmax = P + qlast;                                     // last key any row sees
+  int kmax = P + qlast;                                           // last key any row sees
   const int kmin = window > 0 ? max(0, P + q0 - window + 1) : 0;  // first key any row sees
-  const int kfirst = kmin / kPfKeys * kPfKeys;
+  int kfirst = kmin / kPfKeys * kPfKeys;
+  if constexpr (kSplit) {  // this workgroup's share of the key blocks
+    const int blocks = kmax >= kfirst ? (kmax - kfirst) / kPfKeys + 1 : 0;
+    const int b0 = (int)((int64_t)blocks * share / splits);
+    const int b1 = (int)((int64_t)blocks * (share + 1) / splits);
+    kmax = min(kmax, kfirst + b1 * kPfKeys - 1);
+    kfirst += b0 * kPfKeys;
+  }
 
   // Staging: load j brings page j of the block (keys 16 j .. 16 j + 15),
   // threads 0..127 its K rows, threads 128..255 its V rows, 16-byte part
@@ -862,6 +877,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     lt += __shfl_xor(lt, 16, kWave);
     lt += __shfl_xor(lt, 32, kWave);
     const int qi = q0 + qt * 16 + r;
+    if constexpr (kSplit) {
+      if (qi < qn) {
+        const size_t at = ((size_t)share * rows + qb + qi) * kHq + head;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) *(f32x4*)(part_o + at * kD + dt * 16 + 4 * g) = o[qt][dt];
+        if (g == 0) *(float2*)(part_ml + at * 2) = make_float2(m[qt], lt);
+      }
+      continue;
+    }
     const float lse = (m[qt] + __log2f(lt)) * 0.6931471805599453f;
     const float sf = sink_factor(lse, sinks[head]);
     const float inv = 1.0f / lt;
@@ -876,6 +900,55 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
             make_uint2((uint32_t)v4[0] | ((uint32_t)v4[1] << 16), (uint32_t)v4[2] | ((uint32_t)v4[3] << 16));
       }
     }
+  }
+}
+
+// The shares of a split prefill merged: o and l at the largest reference point,
+// then the epilogue of prefill_kernel.  Workgroup (four rows of a query tile, 4
+// heads); a thread takes four dimensions of a row and head, with every share's
+// loads in flight at once (kMost of them: the splits rounded up).  Bound by the
+// bytes of the partials (mostly in the last-level cache).
+template <int kMost>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(
+    const int* __restrict__ q_indptr, int tiles_per_seq, const uint16_t* __restrict__ sinks,
+    int splits, int rows, const float* __restrict__ part_o, const float* __restrict__ part_ml,
+    uint16_t* __restrict__ out) {
+  constexpr int kRounds = kPfQ / 4;
+  const int tile = blockIdx.x / kRounds;
+  const int b = tile / tiles_per_seq;
+  const int qi = tile % tiles_per_seq * kPfQ + (int)(blockIdx.x % kRounds) * 4 + (threadIdx.x >> 6);
+  const int qb = q_indptr[b], qn = q_indptr[b + 1] - qb;
+  const int t = threadIdx.x, d = (t & 15) * 4, head = blockIdx.y * 4 + (t >> 4 & 3);
+  const uint16_t sink = sinks[head];
+  if (qi < qn) {
+    const size_t at = (size_t)(qb + qi) * kHq + head, step = (size_t)rows * kHq;
+    float2 ml[kMost];
+    f32x4 po[kMost];
+#pragma unroll
+    for (int s = 0; s < kMost; ++s) {  // (past the splits: the last one again, not used)
+      const size_t a = at + (size_t)min(s, splits - 1) * step;
+      ml[s] = *(const float2*)(part_ml + a * 2);
+      po[s] = *(const f32x4*)(part_o + a * kD + d);
+    }
+    float m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int s = 0; s < kMost; ++s) m = s < splits ? fmaxf(m, ml[s].x) : m;
+    f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < kMost; ++s) {
+      // a share with none of the row's keys has m = -inf, l = 0 and o = 0
+      const float w = s < splits && ml[s].x != -INFINITY ? __builtin_amdgcn_exp2f(ml[s].x - m) : 0.f;
+      l = fmaf(ml[s].y, w, l);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = fmaf(po[s][i], w, o[i]);
+    }
+    const float lse = (m + __log2f(l)) * 0.6931471805599453f;
+    const float sf = sink_factor(lse, sink), inv = 1.0f / l;
+    uint16_t v4[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v4[i] = f2bf(bf2f(f2bf(o[i] * inv)) * sf);
+    *(uint2*)(out + at * kD + d) =
+        make_uint2((uint32_t)v4[0] | ((uint32_t)v4[1] << 16), (uint32_t)v4[2] | ((uint32_t)v4[3] << 16));
   }
 }
 
@@ -962,17 +1035,34 @@ int attn_launch_decode(const void* q, int batch, const void* cache, const int* p
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 
+// splits > 1: part_o [splits][rows][64][64], part_ml [splits][rows][64][2] fp32
 int attn_launch_prefill(const void* q, const int* q_indptr, int batch, int max_q_len,
                         const void* cache, const int* page_indptr, const int* page_indices,
                         int num_pages, const int* kv_len, int window, float sm_scale,
-                        const void* sinks, void* out, hipStream_t s) {
+                        const void* sinks, void* out, int splits, int rows, float* part_o,
+                        float* part_ml, hipStream_t s) {
   const int tiles = (max_q_len + attn::kPfQ - 1) / attn::kPfQ;
-  hipLaunchKernelGGL(attn::prefill_kernel, dim3(tiles * batch, attn::kHkv * attn::kPfHalves),
-                     dim3(64 * attn::kPfWaves), 0, s,
-                     (const uint16_t*)q, q_indptr, (const uint8_t*)cache, page_indptr, page_indices,
-                     num_pages, kv_len, window, sm_scale, (const uint16_t*)sinks, tiles,
-                     (uint16_t*)out);
-  return hipGetLastError() == hipSuccess ? 0 : -6;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(tiles * batch * splits, attn::kHkv * attn::kPfHalves),
+                       dim3(64 * attn::kPfWaves), 0, s, (const uint16_t*)q, q_indptr,
+                       (const uint8_t*)cache, page_indptr, page_indices, num_pages, kv_len, window,
+                       sm_scale, (const uint16_t*)sinks, tiles, (uint16_t*)out, splits, rows,
+                       part_o, part_ml);
+    return hipGetLastError() == hipSuccess ? 0 : -6;
+  };
+  if (splits <= 1) return go(attn::prefill_kernel<false>);
+  const int rc = go(attn::prefill_kernel<true>);
+  if (rc) return rc;
+  auto merge = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(tiles * batch * (attn::kPfQ / 4), attn::kHq / 4), dim3(256), 0,
+                       s, q_indptr, tiles, (const uint16_t*)sinks, splits, rows, part_o, part_ml,
+                       (uint16_t*)out);
+    return hipGetLastError() == hipSuccess ? 0 : -6;
+  };
+  return splits <= 2   ? merge(attn::prefill_merge_kernel<2>)
+         : splits <= 4 ? merge(attn::prefill_merge_kernel<4>)
+         : splits <= 8 ? merge(attn::prefill_merge_kernel<8>)
+                       : merge(attn::prefill_merge_kernel<16>);
 }
 
 int attn_launch_bias_residual(const void* x, const void* y, const void* bias, int64_t n, int H,

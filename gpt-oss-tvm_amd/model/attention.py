@@ -156,7 +156,8 @@ class AttentionBlock(torch.nn.Module):
                      window, self.sm_scale, self.sinks, o, ws)
         else:
             A.prefill(q, tables.q_indptr, tables.max_q_len, layer, tables.page_indptr,
-                      tables.page_indices, tables.kv_len, window, self.sm_scale, self.sinks, o)
+                      tables.page_indices, tables.kv_len, window, self.sm_scale, self.sinks, o,
+                      tables.max_kv_len)
         o2 = o.view(n, A.Q_HEADS * A.HEAD_DIM)
         if small:
             return A.rows_bias_residual(o2, self.out.weight, self.out.bias, x2).view(x.shape)

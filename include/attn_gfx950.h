@@ -86,6 +86,21 @@ MOE_API int attn_prefill(const uint16_t* q, const int32_t* q_indptr, int64_t bat
                          const int32_t* kv_len, int32_t window, float sm_scale,
                          const uint16_t* sinks, uint16_t* out, moe_stream_t stream);
 
+/* attn_prefill for calls whose query tiles would not fill the chip (a short text
+ * over a long cached prefix): each tile's keys are shared out over several
+ * workgroups, whose partial results wait in `workspace` (q has `rows` rows, max_kv_len
+ * bounds kv_len and only chooses the split).  attn_prefill_workspace_bytes is 0
+ * where the plain form is taken; the workspace needs no initialisation. */
+MOE_API size_t attn_prefill_workspace_bytes(int64_t rows, int64_t batch, int64_t max_q_len,
+                                            int64_t max_kv_len, int32_t window);
+MOE_API int attn_prefill_split(const uint16_t* q, int64_t rows, const int32_t* q_indptr,
+                               int64_t batch, int64_t max_q_len, const void* kv_cache,
+                               int64_t num_pages, const int32_t* page_indptr,
+                               const int32_t* page_indices, const int32_t* kv_len,
+                               int64_t max_kv_len, int32_t window, float sm_scale,
+                               const uint16_t* sinks, uint16_t* out, void* workspace,
+                               size_t workspace_bytes, moe_stream_t stream);
+
 /* out = bf16(x + bf16(y + bias)): the output nn.Linear's bias add and the
  * residual of model/attention.py:254-256.  x, y, out [n, H]; H % 4 == 0. */
 MOE_API int attn_bias_residual(const uint16_t* x, const uint16_t* y, const uint16_t* bias,

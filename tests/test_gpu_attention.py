@@ -481,3 +481,31 @@ def test_qkv_rope_append_many_tokens(A, n):
     c = host_bf16(cache).transpose(0, 3, 1, 2, 4).reshape(-1, 2, HKV, D)
     np.testing.assert_array_equal(c[slots, 0], AO.rope(rk, pos))
     np.testing.assert_array_equal(c[slots, 1], rv)
+
+
+@pytest.mark.parametrize("qlens,prefix,bound", [
+    ([9], [700], None), ([1, 64, 65, 130], [900, 0, 37, 300], None),
+    ([70], [3000], None),            # 15 shares of three or four key blocks
+    ([300], [500], 4000),            # a bound above the length: shares without keys
+    ([40], [1200], 500)])            # and below it: fewer shares, the same result
+def test_prefill_attention_shared_keys(A, qlens, prefix, bound):
+    """Few query tiles over many keys: the keys shared out over workgroups and
+    merged, for ragged sequences (some with fewer keys than shares), causal
+    rows that see nothing of a share, and any bound."""
+    lengths = [p + q for p, q in zip(prefix, qlens)]
+    bound = bound or max(lengths)
+    n = sum(qlens)
+    assert A._lib.attn_prefill_workspace_bytes(n, len(qlens), max(qlens), bound, 0) > 0
+    seqs = PagedSeqs(91 + n, lengths)
+    rng = np.random.default_rng(92 + n)
+    q = bf(2.0 * rng.standard_normal((n, HQ, D)))
+    sinks = bf(rng.standard_normal(HQ))
+    q_indptr = np.concatenate([[0], np.cumsum(qlens)]).astype(np.int32)
+    out = torch.empty((n, HQ, D), dtype=torch.bfloat16, device="cuda")
+    A.prefill(bf16_dev(q), i32_dev(q_indptr), max(qlens), seqs.cache, seqs.page_indptr,
+              seqs.page_indices, seqs.kv_len, 0, SCALE, bf16_dev(sinks), out, bound)
+    got = host_bf16(out)
+    for b, (L, ql) in enumerate(zip(lengths, qlens)):
+        rows = slice(q_indptr[b], q_indptr[b + 1])
+        o, lse = AO.attention(q[rows], seqs.k[b], seqs.v[b], np.arange(L - ql, L), 0)
+        close(got[rows], AO.sink_scale(o, lse, sinks))
