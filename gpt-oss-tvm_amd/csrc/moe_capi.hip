@@ -95,10 +95,18 @@ int check_dims(int64_t n, int64_t E, int64_t k, int64_t H, int64_t I) {
 inline size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // Expert matmul dispatch (model/mlp_optimized.py:94-107 picks prefill or
-// decode kernels by token count): the tiled GEMM once the experts average
-// kGemmMinTokens or more tokens (each weight tile then serves many tokens),
-// the grouped GEMV below that or when N is not a multiple of its tile.
-constexpr int64_t kGemmMinTokens = 48;
+// decode kernels by token count): the tiled GEMM once the experts average 48 or
+// more pairs (each weight tile then serves many tokens), and above 128 tokens
+// (what the decode launch takes) from 40 on, where the grouped GEMV's token
+// batches overflow and it needs an encoding pass besides; the grouped GEMV below
+// that or when N is not a multiple of the GEMM's tile.  Block us, GEMV / GEMM,
+// uniform routing: 20B at 333 and 383 tokens (41.6 and 47.9 pairs per expert) 217 /
+// 202 and 215 / 205, 120B at 1500 (46.9) 1071 / 707; Zipf: 20B at 383 224 / 220, 120B
+// at 1500 904 / 782.  Lower, skewed routing loses: Zipf at 37.5 pairs 205 / 217
+// (uniform 206 / 178), 120B at 31 667 / 701 (723 / 633).
+bool use_gemm(int64_t pairs, int64_t k, int64_t E) {
+  return pairs >= 48 * E || (pairs > 128 * k && pairs >= 40 * E);
+}
 
 // The decode launch combines a token's k mlp2 rows itself (the last of its k
 // tiles to arrive sums them) up to this many tokens; above it a separate
@@ -138,7 +146,7 @@ int expert_matmul(const void* packed, int rows, int pieces, const int32_t* indpt
                   int max_tokens, int pairs, int swiglu, float alpha, float limit, void* out,
                   int out_ld, hipStream_t s) {
   // the GEMM stores 16-byte row pieces and loads the bias 16 bytes at a time
-  if ((int64_t)pairs >= kGemmMinTokens * E && ((uintptr_t)out & 15u) == 0 && out_ld % 4 == 0 &&
+  if (use_gemm(pairs, k_top, E) && ((uintptr_t)out & 15u) == 0 && out_ld % 4 == 0 &&
       ((uintptr_t)bias & 15u) == 0) {
     const int rc = moe_launch_mx_gemm(packed, rows, pieces, indptr, sorted_pairs, k_top,
                                       arow_mode, orow_mode, blocks, scales, bias, E, N, K, pairs,
@@ -208,8 +216,7 @@ void layout(int64_t n, int64_t E, int64_t k, int64_t H, int64_t I, size_t off[kN
 }
 
 // mlp1 + SwiGLU with act written as its three fp8 pieces (rows by sorted
-// position).  With the tiled GEMM (48 or more pairs per expert on average)
-// the epilogue encodes act directly (a 192-column tile holds whole
+// position).  With the tiled GEMM (use_gemm) the epilogue encodes act directly (a 192-column tile holds whole
 // 32-element blocks of act): no fp32 act round trip and no encoding pass.
 // Otherwise the grouped GEMV writes fp32 act and the pieces kernel encodes it.
 int mlp1_pieces(const void* t_pk, int64_t n, int64_t k, int64_t E, int64_t H, int64_t I,
@@ -218,7 +225,7 @@ int mlp1_pieces(const void* t_pk, int64_t n, int64_t k, int64_t E, int64_t H, in
                 hipStream_t s) {
   const int nk = (int)(n * k);
   int rc;
-  if ((int64_t)nk >= kGemmMinTokens * E && ((uintptr_t)bias & 15u) == 0) {
+  if (use_gemm(nk, k, E) && ((uintptr_t)bias & 15u) == 0) {
     rc = moe_launch_mx_gemm(t_pk, (int)n, kPiecesT, indptr, sp, (int)k, 0, 1, blocks, scales,
                             bias, (int)E, (int)(2 * I), (int)H, nk, 2, alpha, limit, act_pk,
                             (int)I, (char*)act_pk + moe_pieces_q_bytes(nk, I, kPiecesAct), s);
@@ -520,7 +527,7 @@ static int block_forward_impl(const uint16_t* x, int64_t n, int64_t E, int64_t k
   float* logits = (float*)(ws + off[12]);
   int32_t* counts = (int32_t*)(ws + off[13]);
   int32_t* sync = (int32_t*)(ws + off[kRegionSync]);  // [E] counts, [E] status
-  const bool gemm = (int64_t)nk >= kGemmMinTokens * E;
+  const bool gemm = use_gemm(nk, k, E);
   // norm, t, its pieces and the logits (and sync[0..E] = 0: the decode
   // launch's counts and status); then top-k, softmax and grouping
   void* t_qs = (char*)t_pk + moe_pieces_q_bytes(n, H, kPiecesT);

@@ -6,16 +6,24 @@
 // (model/mlp_optimized.py:214-460) with the fp32 semantics of
 // model/mlp.py:387-395 (einsum + bias, interleaved clamped SwiGLU on mlp1).
 //
-// Tiles.  A work unit is one (expert, token tile, column tile): 192 A rows
-// (192 / P tokens, P pieces each) against 192 weight rows over the whole K.
-// Eight waves split it 4 x 2: each wave owns 48 A rows x 96 columns, i.e.
-// 3 x 6 MFMA tiles of 16 x 16, and keeps their 18 accumulators for all of K.
+// Tiles.  A work unit is one (expert, token tile, column tile): kRows A rows
+// (kRows / P tokens, P pieces each) against 192 weight rows over the whole K.
+// With 192 rows eight waves split it 4 x 2, with 96 rows four waves 2 x 2: each
+// wave owns 48 A rows x 96 columns, i.e. 3 x 6 MFMA tiles of 16 x 16, and keeps
+// their 18 accumulators for all of K.
+//   192 rows: one workgroup per CU, three code stages.  The direct loads bind it
+//     (without them the K loop's time falls by a quarter; without its MFMAs, its
+//     operand reads or its scale reads by 0 to 5%), so the large tile is the one
+//     for many tokens: 96 rows load a third more per product.
+//   96 rows (mlp1): two workgroups per CU, two stages, for experts of fewer than 48
+//     pairs on average, where a unit's time is its chain of loads and the last, partly
+//     filled tiles weigh most (launch_rows has the figures).
 //
 // Staging.  The unit's scale bytes (A: 112 per row, B: G per column) are
 // staged once.  Per 128-wide K chunk a stage holds the tile's A codes
-// (192 x 128 bytes) and B codes (192 x 64).  Both come by direct
-// global-to-LDS loads (no registers), 16 bytes per lane; three code stages
-// form a ring, so while chunk c is multiplied the loads of chunks c + 1 and
+// (kRows x 128 bytes) and B codes (192 x 64).  Both come by direct
+// global-to-LDS loads (no registers), 16 bytes per lane; the code stages form a
+// ring: with three, while chunk c is multiplied the loads of chunks c + 1 and
 // c + 2 are in flight.  A wave's loads complete in issue order, so "chunk c
 // has landed" is vmcnt <= (its loads per chunk) on each wave plus a barrier.
 // A and B code rows are stored with their 16-byte parts XOR-swizzled so that
@@ -28,38 +36,44 @@
 //   D  column r, elements i = 0..3 -> A rows 4 g + i
 // A token's P piece rows share one lane's four accumulator rows, so the
 // pieces are summed in registers in the epilogue, as the GEMV does.
+#include <algorithm>
 #include <type_traits>
 
 #include "moe_common.h"
 
 namespace moe {
 
-constexpr int kGmRows = 192;                       // A rows per tile
 constexpr int kGmCols = 192;                       // weight rows (output columns) per tile
-constexpr int kGmWaves = 8;                        // 4 (A rows) x 2 (columns)
-constexpr int kGmThreads = 64 * kGmWaves;
-constexpr int kGmStages = 3;
-constexpr int kGmAInst = kGmRows * 8 / 64;         // 24 A-code loads per chunk (3 per wave)
 constexpr int kGmBInst = kGmCols * 4 / 64;         // 12 B-code loads per chunk
-constexpr int kGmAo = 0;                           // in a stage: A codes, then B codes
-constexpr int kGmBo = kGmRows * 128;
-constexpr int kGmStage = kGmBo + kGmCols * 64;     // 36864 bytes
 constexpr int kGmSclRow = 112;                     // scale bytes per piece row (4 runs of 28)
 constexpr int kGmMaxG = 96;                        // K <= 3072
-constexpr int kGmASc = kGmStages * kGmStage;       // A scales of the unit [rows][112]
-constexpr int kGmBSc = kGmASc + kGmRows * kGmSclRow;  // B scales of the unit [cols][G]
-constexpr int kGmBScBytes = kGmCols * kGmMaxG;     // 192 G, G <= 96, in whole 1 KB loads
-constexpr int kGmBias = kGmBSc + kGmBScBytes;      // bias of the unit's columns (bf16)
-constexpr int kGmFixedLds = kGmBias + 1024;        // 152064 bytes
 constexpr int kGmCUs = 256;                        // MI355X
 constexpr int kGmXcds = 8;                         // 8 XCDs of 32 CUs, one L2 each
 
-// dynamic part: unit prefix and indptr, E + 1 ints each
-// dynamic part: unit prefix and indptr, E + 1 ints each, then two buffers of
-// a unit's sorted_pairs entries (kGmSpMax ints each)
-constexpr int kGmSpMax = kGmRows / 2;
-__host__ __device__ constexpr int gm_lds_bytes(int E) { return 2 * (E + 1) * 4 + 2 * kGmSpMax * 4; }
-static_assert(kGmFixedLds + gm_lds_bytes(256) <= 160 * 1024, "LDS");
+// A tile of kRows A rows: waves, stages and the static LDS (byte offsets)
+template <int kRows>
+struct Gm {
+  static constexpr int wave_rows = kRows / 48;     // waves along the A rows (x 2 column halves)
+  static constexpr int waves = 2 * wave_rows;
+  static constexpr int threads = 64 * waves;
+  static constexpr int per_cu = kRows == 192 ? 1 : 2;  // workgroups of a CU
+  static constexpr int stages = kRows == 192 ? 3 : 2;
+  static constexpr int b_wave = (kGmBInst + waves - 1) / waves;  // B-code loads of a wave
+  static constexpr int ao = 0;                     // in a stage: A codes, then B codes
+  static constexpr int bo = kRows * 128;
+  static constexpr int stage = bo + kGmCols * 64;
+  // scales of the unit, A [rows][112] and B [cols][G], in whole 1 KB loads
+  static constexpr int asc = stages * stage;
+  static constexpr int bsc = asc + (kRows * kGmSclRow + 1023) / 1024 * 1024;
+  static constexpr int bias = bsc + kGmCols * kGmMaxG;  // bias of the unit's columns (bf16)
+  static constexpr int bytes = bias + 1024;
+  // dynamic part: unit prefix and indptr, E + 1 ints each, then two buffers of
+  // a unit's rows (activation and output row of each token, sp_max ints each)
+  static constexpr int sp_max = kRows / 2;
+  static constexpr int dyn_bytes(int E) { return 2 * (E + 1) * 4 + 4 * sp_max * 4; }
+};
+static_assert(Gm<192>::bytes + Gm<192>::dyn_bytes(256) <= 160 * 1024, "LDS");
+static_assert(2 * (Gm<96>::bytes + Gm<96>::dyn_bytes(128)) <= 160 * 1024, "two per CU");
 
 
 template <int S, int E, class F>
@@ -105,50 +119,56 @@ __device__ __forceinline__ float gm_row_down(float x, float y, int g) {
   return __int_as_float(g == 1 ? (int)a[0] : g == 3 ? (int)c[0] : (int)s16[1]);
 }
 
-template <int P, int kEpi>
-__global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
+template <int P, int kEpi, int kRows>
+__global__ __launch_bounds__(Gm<kRows>::threads, 2) void moe_mx_gemm_kernel(
     const uint8_t* __restrict__ q, const uint8_t* __restrict__ qs, int Kp,
     const int* __restrict__ indptr, const int* __restrict__ sorted_pairs, int k_top,
     int arow_mode, int orow_mode, const uint8_t* __restrict__ blocks,
     const uint8_t* __restrict__ scales, const uint16_t* __restrict__ bias, int N, int G, int E,
     float alpha, float limit, float* __restrict__ out, int out_ld, int xcds,
     uint8_t* __restrict__ oqs) {
-  __shared__ __align__(16) uint8_t ring[kGmFixedLds];
+  using C = Gm<kRows>;
+  __shared__ __align__(16) uint8_t ring[C::bytes];
   extern __shared__ __align__(16) uint8_t lds[];  // unit prefix
-  constexpr int TPT = kGmRows / P;  // tokens per tile
+  constexpr int TPT = kRows / P;  // tokens per tile
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 3, wn = wave >> 2;
+  const int wm = wave % C::wave_rows, wn = wave / C::wave_rows;
   const int r = lane & 15, g = lane >> 4;
   const int NT = N / kGmCols;
   const int NC = Kp >> 7;
-  // B-code loads per chunk: instruction k < 12 belongs to wave k % 8
-  const bool two_b = wave < kGmBInst - kGmWaves;
+  // B-code loads per chunk: instruction k < 12 belongs to wave k % waves
+  const bool last_b = wave + C::waves * (C::b_wave - 1) < kGmBInst;
   // Per-lane LDS read bases of each stage; the operand index goes into the
   // instructions' immediate offsets.  Lane (r, g): B column 96 wn + 16 b + r
   // (part g, swizzled by (column >> 1) & 3 = (r >> 1) & 3); A row
   // 48 wm + 16 f + r (parts g and g + 4, swizzled by row & 7 = r & 7).
   const uint32_t rbase = lds_addr(ring);
-  uint32_t vb[kGmStages], va0[kGmStages], va1[kGmStages];
+  uint32_t vb[C::stages], va0[C::stages], va1[C::stages];
 #pragma unroll
-  for (int S = 0; S < kGmStages; ++S) {
-    const uint32_t st = rbase + S * kGmStage;
-    vb[S] = st + kGmBo + (96 * wn + r) * 64 + ((g ^ ((r >> 1) & 3)) << 4);
-    va0[S] = st + kGmAo + (48 * wm + r) * 128 + ((g ^ (r & 7)) << 4);
-    va1[S] = st + kGmAo + (48 * wm + r) * 128 + (((g + 4) ^ (r & 7)) << 4);
+  for (int S = 0; S < C::stages; ++S) {
+    const uint32_t st = rbase + S * C::stage;
+    vb[S] = st + C::bo + (96 * wn + r) * 64 + ((g ^ ((r >> 1) & 3)) << 4);
+    va0[S] = st + C::ao + (48 * wm + r) * 128 + ((g ^ (r & 7)) << 4);
+    va1[S] = st + C::ao + (48 * wm + r) * 128 + (((g + 4) ^ (r & 7)) << 4);
   }
   // scale bytes: A row 48 wm + 16 f + r, run g; B column 96 wn + 16 b + r
-  const uint32_t vas = rbase + kGmASc + (48 * wm + r) * kGmSclRow + g * 28;
-  const uint32_t vbs = rbase + kGmBSc + (96 * wn + r) * G;
+  const uint32_t vas = rbase + C::asc + (48 * wm + r) * kGmSclRow + g * 28;
+  const uint32_t vbs = rbase + C::bsc + (96 * wn + r) * G;
   int* const pre = (int*)lds;
   int* const ipl = pre + (E + 1);  // indptr, read once
-  // A unit's sorted_pairs entries (token tt at [tt]) in LDS, double-buffered:
-  // each unit's epilogue loads the next unit's before any of its stores, so
-  // no global load in the address chains or the stores waits behind stores
-  // (vmcnt counts loads and stores together, in issue order).
+  // A unit's rows in LDS (token tt's activation row at [tt], its output row at
+  // [C::sp_max + tt]), double-buffered: each unit's epilogue loads the next unit's
+  // sorted_pairs entries before any of its stores, so no global load in the
+  // address chains or the stores waits behind stores (vmcnt counts loads and
+  // stores together, in issue order).
   int* const spb = ipl + (E + 1);
   const bool need_sp = arow_mode != 2 || orow_mode == 0;
+  auto put_rows = [&](int* sp, int tt, int pair, int j) {
+    sp[tt] = arow_mode == 0 ? pair / k_top : arow_mode == 1 ? pair : j;
+    sp[C::sp_max + tt] = orow_mode == 0 ? pair : j;
+  };
   int par = 0;
   bool first_unit = true;
 
@@ -179,15 +199,15 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
   const int vwg = xcds > 1 ? (int)(blockIdx.x % xcds) * (int)(gridDim.x / xcds) +
                                  (int)(blockIdx.x / xcds)
                            : (int)blockIdx.x;
-  auto expert_of = [&](int u) {  // largest e with pre[e] <= u
-    int lo = 0, hi = E - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (pre[mid] <= u) lo = mid; else hi = mid - 1;
-    }
-    return lo;
+  // The expert of unit u (the largest e with pre[e] <= u), searched on from the
+  // workgroup's last one: its units ascend.  Wave-uniform, in a scalar register, so
+  // that the unit's indices and base addresses are scalar arithmetic too.
+  int e_at = 0;
+  auto expert_of = [&](int u) {
+    while (e_at < E - 1 && __builtin_amdgcn_readfirstlane(pre[e_at + 1]) <= u) ++e_at;
+    return e_at;
   };
-
+  auto uni = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
   for (int u = vwg; u < total; u += gridDim.x) {
     // An opaque copy of the lane index for this unit's address arithmetic:
     // the compiler would otherwise hoist lane-dependent addresses out of the
@@ -196,94 +216,93 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
     int lane_u = lane;
     asm volatile("" : "+v"(lane_u));
     const int e = expert_of(u);
-    const int off = u - pre[e];
+    const int off = u - uni(pre[e]);
     const int mt = off / NT, nt = off - mt * NT;
-    const int start = ipl[e];
+    const int start = uni(ipl[e]);
     const int m0 = mt * TPT;
-    const int ntok = min(TPT, ipl[e + 1] - start - m0);
+    const int ntok = min(TPT, uni(ipl[e + 1]) - start - m0);
     const int n0 = nt * kGmCols;
-    int* const spu = spb + par * kGmSpMax;
-    if (need_sp && first_unit) {
-      if (tid < ntok) spu[tid] = sorted_pairs[start + m0 + tid];
+    int* const spu = spb + par * 2 * C::sp_max;
+    if (first_unit) {
+      if (tid < ntok)
+        put_rows(spu, tid, need_sp ? sorted_pairs[start + m0 + tid] : 0, start + m0 + tid);
       __syncthreads();  // (the first unit: nothing else in flight)
     }
     first_unit = false;
-    auto src_row = [&](int tt) {  // activation row of token tt of this tile
-      return arow_mode == 0 ? spu[tt] / k_top : arow_mode == 1 ? spu[tt] : start + m0 + tt;
-    };
     // Rows past the tile's tokens load token 0's row: their MFMA rows are
     // computed and never stored (a D row depends on its A row only).
     auto piece_row = [&](int R) {  // packed-pieces row of tile A row R
       if constexpr (P == 3) asm volatile("" : "+v"(R));  // (not hoisted: see the epilogue)
       const int tt = R / P, p = R - tt * P;
-      return (uint32_t)(src_row(tt < ntok ? tt : 0) * P + p);
+      return (uint32_t)(spu[tt < ntok ? tt : 0] * P + p);
     };
 
     // The unit's scales, 16 bytes per lane_u: A rows (7 loads of 16 per row;
     // loads past the last row repeat it), then the B columns' G bytes each
     // (192 G contiguous checkpoint bytes; the tail repeats the last 16).
     {
-      constexpr int kAU = kGmRows * 7;                        // 1344 A-scale loads
+      constexpr int kAU = kRows * 7;                        // 1344 A-scale loads
       const int nbu = kGmCols * G / 16;                       // B-scale loads
-      for (int i0 = 64 * wave; i0 < kAU; i0 += kGmThreads) {
+      for (int i0 = 64 * wave; i0 < kAU; i0 += C::threads) {
         const int uu = min(i0 + lane_u, kAU - 1), R = uu / 7;
         __builtin_amdgcn_global_load_lds(
             (const void*)(qs + piece_row(R) * kGmSclRow + (uu - R * 7) * 16),
-            (lds_ptr_t)(ring + kGmASc + i0 * 16), 16, 0, 0);
+            (lds_ptr_t)(ring + C::asc + i0 * 16), 16, 0, 0);
       }
       const uint8_t* bsrc = scales + ((size_t)e * N + n0) * G;
-      for (int i0 = 64 * wave; i0 < nbu; i0 += kGmThreads)
+      for (int i0 = 64 * wave; i0 < nbu; i0 += C::threads)
         __builtin_amdgcn_global_load_lds((const void*)(bsrc + min(i0 + lane_u, nbu - 1) * 16),
-                                         (lds_ptr_t)(ring + kGmBSc + i0 * 16), 16, 0, 0);
+                                         (lds_ptr_t)(ring + C::bsc + i0 * 16), 16, 0, 0);
       // the columns' bias: 384 bytes, 24 loads of 16 (the rest repeat the last)
-      if (wave == kGmWaves - 1)
+      if (wave == C::waves - 1)
         __builtin_amdgcn_global_load_lds(
             (const void*)((const uint8_t*)(bias + (size_t)e * N + n0) + min(lane_u, 23) * 16),
-            (lds_ptr_t)(ring + kGmBias), 16, 0, 0);
+            (lds_ptr_t)(ring + C::bias), 16, 0, 0);
     }
 
     // This wave's code loads of a chunk (lane_u l), 32-bit offsets from q and
     // blocks (the launcher checks the ranges):
     //  A 3: instruction 3 w + m, rows 8 (3 w + m) + l / 8, global part
     //       (l % 8) ^ (l / 8)
-    //  B 1 or 2: instruction k = w (+ 8), columns 16 k + l / 4, global part
+    //  B b_wave (or one less): instruction k = w + waves m, columns 16 k + l / 4, global part
     //       (l % 4) ^ ((column >> 1) & 3)
-    uint32_t ap[3], bp[2];
-    int bpart[2];
+    uint32_t ap[3], bp[C::b_wave];
+    int bpart[C::b_wave];
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
       const int R = 8 * (3 * wave + m) + (lane_u >> 3);
       ap[m] = piece_row(R) * (uint32_t)Kp + (((lane_u & 7) ^ (lane_u >> 3)) << 4);
     }
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      const int C = 16 * (wave + kGmWaves * m) + (lane_u >> 2);
-      bp[m] = (uint32_t)(((size_t)e * N + n0 + min(C, kGmCols - 1)) * G * 16);
-      bpart[m] = (lane_u & 3) ^ ((C >> 1) & 3);
+    for (int m = 0; m < C::b_wave; ++m) {
+      const int col = 16 * (wave + C::waves * m) + (lane_u >> 2);
+      bp[m] = (uint32_t)(((size_t)e * N + n0 + min(col, kGmCols - 1)) * G * 16);
+      bpart[m] = (lane_u & 3) ^ ((col >> 1) & 3);
     }
     auto issue_chunk = [&](int c, int S) {
-      uint8_t* st = ring + S * kGmStage;
+      uint8_t* st = ring + S * C::stage;
 #pragma unroll
       for (int m = 0; m < 3; ++m)
         __builtin_amdgcn_global_load_lds((const void*)(q + ap[m] + c * 128),
-                                         (lds_ptr_t)(st + kGmAo + (3 * wave + m) * 1024), 16, 0,
+                                         (lds_ptr_t)(st + C::ao + (3 * wave + m) * 1024), 16, 0,
                                          0);
 #pragma unroll
-      for (int m = 0; m < 2; ++m) {
-        if (m == 0 || two_b) {
+      for (int m = 0; m < C::b_wave; ++m) {
+        if (m < C::b_wave - 1 || last_b) {
           // past K a column re-reads block G - 1 (finite; its A codes are zero)
           const uint32_t blk = (uint32_t)min(4 * c + bpart[m], G - 1);
           __builtin_amdgcn_global_load_lds((const void*)(blocks + bp[m] + blk * 16),
-                                           (lds_ptr_t)(st + kGmBo + (wave + kGmWaves * m) * 1024),
+                                           (lds_ptr_t)(st + C::bo + (wave + C::waves * m) * 1024),
                                            16, 0, 0);
         }
       }
     };
 
-    // Chunks 0..2 in flight; chunk 0's operands go to registers first.
+    // Every stage in flight; chunk 0's operands go to registers first.
     issue_chunk(0, 0);
     if (NC > 1) issue_chunk(1, 1);
-    if (NC > 2) issue_chunk(2, 2);
+    if constexpr (C::stages == 3)
+      if (NC > 2) issue_chunk(2, 2);
 
     f32x4 acc[3][6];
 #pragma unroll
@@ -341,19 +360,21 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
     };
 
     // wait until at most `pending` later chunks' loads are outstanding (a
-    // wave issues 4 or 5 loads per chunk; its loads complete in order)
+    // wave's loads per chunk: 3 of A and b_wave, or one less, of B; its loads
+    // complete in order)
     auto wait_chunks = [&](int pending) {
+      constexpr int kL = 3 + C::b_wave;
       if (pending >= 2) {
-        if (two_b) wait_vmcnt<10>(); else wait_vmcnt<8>();
+        if (last_b) wait_vmcnt<2 * kL>(); else wait_vmcnt<2 * (kL - 1)>();
       } else if (pending == 1) {
-        if (two_b) wait_vmcnt<5>(); else wait_vmcnt<4>();
+        if (last_b) wait_vmcnt<kL>(); else wait_vmcnt<kL - 1>();
       } else {
         wait_vmcnt<0>();
       }
     };
     Ops cur, nxt;
     // chunk 0 landed (and the unit's scales: issued before it)
-    wait_chunks(min(NC - 1, 2));
+    wait_chunks(min(NC - 1, C::stages - 1));
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     read_b(cur, 0, std::integral_constant<int, 0>{});
@@ -370,20 +391,26 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
     // operand reads, six more MFMAs, then the chunk loads and the other A
     // reads, the last six MFMAs.  (Measured against the loads and reads
     // ahead of the MFMAs, and against one MFMA between each pair of memory
-    // instructions: both are slower.)
+    // instructions: both are slower.)  With two stages chunk c + 2 is issued
+    // instead, straight after the barrier, and the other workgroup of the CU
+    // covers the waits.
     auto step = [&](int c, Ops& cu, Ops& nx, auto sv) {
       constexpr int S = decltype(sv)::value;           // stage of chunk c
-      constexpr int S1 = (S + 1) % kGmStages;          // stage of chunk c + 1
+      constexpr int S1 = (S + 1) % C::stages;          // stage of chunk c + 1
       const bool more = c + 1 < NC;
       using I0 = std::integral_constant<int, 0>;
       using I1 = std::integral_constant<int, 1>;
       using I2 = std::integral_constant<int, 2>;
       using SS1 = std::integral_constant<int, S1>;
       if (more) {
-        wait_chunks(c + 2 < NC ? 1 : 0);
+        wait_chunks(C::stages == 3 && c + 2 < NC ? 1 : 0);
         __builtin_amdgcn_s_barrier();
       }
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (C::stages == 2) {
+        if (c + 2 < NC) issue_chunk(c + 2, S);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       if (0 < nf) mfma_group(cu, I0{});
       __builtin_amdgcn_sched_barrier(0);
       if (more) {
@@ -394,7 +421,8 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
       if (1 < nf) mfma_group(cu, I1{});
       __builtin_amdgcn_sched_barrier(0);
       if (more) {
-        if (c + 3 < NC) issue_chunk(c + 3, S);
+        if constexpr (C::stages == 3)
+          if (c + 3 < NC) issue_chunk(c + 3, S);
         read_a(nx, c + 1, SS1{}, I1{});
         read_a(nx, c + 1, SS1{}, I2{});
       }
@@ -403,16 +431,17 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
       __builtin_amdgcn_sched_barrier(0);
       if (more) wait_ops(nx);
     };
-    // Register sets alternate with the chunk parity and stages with c % 3,
-    // so the loop is unrolled by six.
-    for (int c = 0; c < NC; c += 6) {
-      step(c, cur, nxt, std::integral_constant<int, 0>{});
-      if (c + 1 < NC) step(c + 1, nxt, cur, std::integral_constant<int, 1>{});
-      if (c + 2 < NC) step(c + 2, cur, nxt, std::integral_constant<int, 2>{});
-      if (c + 3 < NC) step(c + 3, nxt, cur, std::integral_constant<int, 0>{});
-      if (c + 4 < NC) step(c + 4, cur, nxt, std::integral_constant<int, 1>{});
-      if (c + 5 < NC) step(c + 5, nxt, cur, std::integral_constant<int, 2>{});
-    }
+    // Register sets alternate with the chunk parity and stages with c % stages,
+    // so the loop is unrolled by six or two.
+    constexpr int kUnroll = C::stages == 3 ? 6 : 2;
+    for (int c = 0; c < NC; c += kUnroll)
+      gm_static_for<0, kUnroll>([&](auto uv) {
+        constexpr int U = decltype(uv)::value;
+        using SS = std::integral_constant<int, U % C::stages>;
+        if (U == 0 || c + U < NC) {
+          if constexpr (U % 2 == 0) step(c + U, cur, nxt, SS{}); else step(c + U, nxt, cur, SS{});
+        }
+      });
     // The MFMAs combine all 64 lanes; the LDS writes below are per-lane.  The
     // empty asm keeps the compiler from sinking the chains into them.
 #pragma unroll
@@ -422,14 +451,15 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
     // every wave is done with the stages: the output tile reuses them
     __syncthreads();
     // the next unit's sorted_pairs entries, loaded before this unit's stores
-    int spn = 0;
+    int spn = 0, jn = 0;
     bool spn_lane = false;
-    if (need_sp && u + (int)gridDim.x < total) {
+    if (u + (int)gridDim.x < total) {
       const int un = u + (int)gridDim.x;
       const int e2 = expert_of(un);
-      const int st2 = ipl[e2], m02 = (un - pre[e2]) / NT * TPT;
-      if (tid < min(TPT, ipl[e2 + 1] - st2 - m02)) {
-        spn = sorted_pairs[st2 + m02 + tid];
+      const int st2 = uni(ipl[e2]), m02 = (un - uni(pre[e2])) / NT * TPT;
+      if (tid < min(TPT, uni(ipl[e2 + 1]) - st2 - m02)) {
+        jn = st2 + m02 + tid;
+        if (need_sp) spn = sorted_pairs[jn];
         spn_lane = true;
       }
     }
@@ -440,8 +470,8 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
     constexpr int TW = kEpi >= 1 ? kGmCols / 2 : kGmCols;
     constexpr int TWp = TW + 4;
     float* const tile = (float*)ring;
-    static_assert(TPT * TWp * 4 <= kGmStages * kGmStage, "output tile");
-    const uint16_t* const bias_l = (const uint16_t*)(ring + kGmBias);
+    static_assert(TPT * TWp * 4 <= C::stages * C::stage, "output tile");
+    const uint16_t* const bias_l = (const uint16_t*)(ring + C::bias);
     if constexpr (P == 3) {
       // The wave's 48 rows 48 wm + 4 q + i (q = 4 f + g, i < 4) hold 16
       // tokens, row 3 t + p piece p of token t.  Every third quad repeats:
@@ -455,7 +485,7 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
       // and the second token's value of a q % 3 = 0 quad is written by every
       // lane, the others' into the spare row TPT, which is never read.  The
       // exchange is by lane-row swaps (register moves, no LDS round trip).
-      static_assert((TPT + 1) * TWp * 4 <= kGmStages * kGmStage, "spare row");
+      static_assert((TPT + 1) * TWp * 4 <= C::stages * C::stage, "spare row");
 #pragma unroll
       for (int b = 0; b < 6; ++b) {
         const int cl = 96 * wn + 16 * b + r;
@@ -503,11 +533,16 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
             const float xg = fminf(glu, limit);
             const float xl = fminf(fmaxf(lin, -limit), limit);
             const float z = __fmul_rn(alpha, xg);
-            // sigmoid from the hardware exp2 and reciprocal (v_exp_f32 of
-            // -z log2(e), v_rcp_f32: a few ulp of the correctly rounded value;
-            // the epilogue is VALU-bound and the library expf and division
-            // cost about 25 instructions per element)
-            const float sig = __builtin_amdgcn_rcpf(1.0f + __expf(-z));
+            // 192 rows: sigmoid from the hardware exp2 and reciprocal (v_exp_f32
+            // of -z log2(e), v_rcp_f32: a few ulp of the correctly rounded
+            // value; the epilogue is VALU-bound and the library expf and division
+            // cost about 25 instructions per element).  96 rows: the library's,
+            // as the grouped GEMV (the other workgroup's K loop covers it).
+            float sig;
+            if constexpr (kRows == 192)
+              sig = __builtin_amdgcn_rcpf(1.0f + __expf(-z));
+            else
+              sig = 1.0f / (1.0f + expf(-z));
             tile[(tt0 + (odd ? 1 : 0)) * TWp + (cl >> 1)] =
                 __fmul_rn(__fmul_rn(xg, sig), __fadd_rn(xl, 1.0f));
           } else {
@@ -518,7 +553,7 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
       }
     }
     }
-    if (spn_lane) spb[(par ^ 1) * kGmSpMax + tid] = spn;
+    if (spn_lane) put_rows(spb + (par ^ 1) * 2 * C::sp_max, tid, spn, jn);
     __syncthreads();
     if constexpr (kEpi == 2) {
       // SwiGLU output straight into three fp8 pieces (the mlp2 operand), the
@@ -533,7 +568,7 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
       uint8_t* const oq = (uint8_t*)out;
       const int cbase = n0 / 2;
       const int tasks = ntok * 12;
-      for (int i0 = 0; i0 < tasks; i0 += kGmThreads) {
+      for (int i0 = 0; i0 < tasks; i0 += C::threads) {
         const int id = i0 + tid;
         const bool valid = id < tasks;
         const int idc = valid ? id : (id & 3);
@@ -542,7 +577,7 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
         const f32x4 v0 = *(const f32x4*)(tile + tt * TWp + bk * 32 + quarter * 8);
         const f32x4 v1 = *(const f32x4*)(tile + tt * TWp + bk * 32 + quarter * 8 + 4);
         float rr[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-        const int orow = orow_mode == 0 ? spu[tt] : start + m0 + tt;
+        const int orow = spu[C::sp_max + tt];
         const int blk = cbase / 32 + bk, ch = blk >> 2, gg = blk & 3;
 #pragma unroll
         for (int p = 0; p < PO; ++p) {
@@ -567,9 +602,9 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
       // Ka, zero scales for the blocks past Ka and for the runs' unused
       // chunks [NCa, 28).
       if (nt == NT - 1) {
-        for (int rp = tid; rp < ntok * PO; rp += kGmThreads) {
+        for (int rp = tid; rp < ntok * PO; rp += C::threads) {
           const int tt = rp / PO, p = rp - tt * PO;
-          const int orow = orow_mode == 0 ? spu[tt] : start + m0 + tt;
+          const int orow = spu[C::sp_max + tt];
           const size_t prow = (size_t)orow * PO + p;
           for (int c = Ka; c < Kpa; c += 16) *(u32x4*)(oq + prow * Kpa + c) = u32x4{0u, 0u, 0u, 0u};
           uint8_t* const run = oqs + prow * kGmSclRow;
@@ -581,10 +616,9 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
     } else {
       constexpr int U = TW / 4;  // 16-byte units per row
       const int cbase = kEpi == 1 ? n0 / 2 : n0;
-      for (int uu = tid; uu < ntok * U; uu += kGmThreads) {
+      for (int uu = tid; uu < ntok * U; uu += C::threads) {
         const int row = uu / U, cu4 = uu - row * U;
-        const int j = start + m0 + row;
-        const int orow = orow_mode == 0 ? spu[row] : j;
+        const int orow = spu[C::sp_max + row];
         *(f32x4*)(out + (size_t)orow * out_ld + cbase + 4 * cu4) =
             *(const f32x4*)(tile + row * TWp + 4 * cu4);
       }
@@ -599,21 +633,38 @@ __global__ __launch_bounds__(kGmThreads) void moe_mx_gemm_kernel(
   }
 }
 
-template <int P, int kEpi>
-int launch_gm(dim3 grid, size_t lds, hipStream_t stream, const uint8_t* q, const uint8_t* qs,
-              int Kp, const int* indptr, const int* sp, int k_top, int arow, int orow,
+template <int P, int kEpi, int kRows>
+int launch_gm(int64_t rows_active, hipStream_t stream, const uint8_t* q, const uint8_t* qs, int Kp,
+              const int* indptr, const int* sp, int k_top, int arow, int orow,
               const uint8_t* blocks, const uint8_t* scales, const uint16_t* bias, int N, int G,
-              int E, float alpha, float limit, float* out, int out_ld, int xcds, uint8_t* oqs) {
-  static const bool lds_ok = [] {  // more than 64 KB of dynamic LDS, once per kernel
-    return hipFuncSetAttribute((const void*)moe_mx_gemm_kernel<P, kEpi>,
+              int E, float alpha, float limit, float* out, int out_ld, uint8_t* oqs) {
+  using C = Gm<kRows>;
+  static const bool lds_ok = [] {  // more than 64 KB of LDS, once per kernel
+    return hipFuncSetAttribute((const void*)moe_mx_gemm_kernel<P, kEpi, kRows>,
                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                               gm_lds_bytes(256)) == hipSuccess;
+                               C::dyn_bytes(256)) == hipSuccess;
   }();
   if (!lds_ok) return kErrLaunch;
-  hipLaunchKernelGGL((moe_mx_gemm_kernel<P, kEpi>), grid, dim3(kGmThreads), lds, stream, q, qs,
-                     Kp, indptr, sp, k_top, arow, orow, blocks, scales, bias, N, G, E, alpha,
-                     limit, out, out_ld, xcds, oqs);
+  const int64_t units_max = (int64_t)(N / kGmCols) * (std::max<int64_t>(1, std::min<int64_t>(E, rows_active)) +
+                                                      rows_active / (kRows / P));
+  if (units_max >= ((int64_t)1 << 31)) return kErrUnsupported;
+  const int nwg = (int)std::min<int64_t>(units_max, C::per_cu * kGmCUs);
+  const int xcds = nwg % kGmXcds == 0 ? kGmXcds : 1;
+  hipLaunchKernelGGL((moe_mx_gemm_kernel<P, kEpi, kRows>), dim3(nwg), dim3(C::threads),
+                     C::dyn_bytes(E), stream, q, qs, Kp, indptr, sp, k_top, arow, orow, blocks,
+                     scales, bias, N, G, E, alpha, limit, out, out_ld, xcds, oqs);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
+// Rows of a tile: 96 for two pieces (mlp1) below 48 pairs per expert on average (its
+// 48 tokens then hold most experts), else 192.  mlp1 us per launch with 96 / 192
+// rows, 20B at 333 and 383 tokens uniform 119 / 113 and 120 / 115, at 383 with Zipf
+// routing 115 / 134; 120B at 1500 uniform 405 / 407, Zipf 431 / 465.
+template <int P, int kEpi, class... A>
+int launch_rows(int64_t rows_active, int E, A... args) {
+  if constexpr (P == 2)
+    if (rows_active < (int64_t)48 * E) return launch_gm<P, kEpi, 96>(rows_active, args...);
+  return launch_gm<P, kEpi, 192>(rows_active, args...);
 }
 
 }  // namespace moe
@@ -639,38 +690,29 @@ int moe_launch_mx_gemm(const void* packed, int rows, int pieces, const void* ind
   const int NC = (K + 127) / 128, Kp = NC * 128, G = K / 32;
   const uint8_t* q = (const uint8_t*)packed;
   const uint8_t* qs = q + moe_pieces_q_bytes(rows, K, pieces);
-  const int tpt = moe::kGmRows / pieces;
-  const int64_t units_max = (int64_t)(N / moe::kGmCols) *
-                            ((int64_t)max(1, min(E, rows_active)) + rows_active / tpt);
-  if (units_max >= ((int64_t)1 << 31)) return moe::kErrUnsupported;
-  const int nwg = (int)(units_max < moe::kGmCUs ? units_max : moe::kGmCUs);
-  const int xcds = nwg % moe::kGmXcds == 0 ? moe::kGmXcds : 1;
-  const size_t lds = moe::gm_lds_bytes(E);
   const int* ip = (const int*)indptr;
   const int* sp = (const int*)sorted_pairs;
   const uint8_t* b = (const uint8_t*)blocks;
   const uint8_t* s = (const uint8_t*)scales;
   const uint16_t* bi = (const uint16_t*)bias;
   float* o = (float*)out;
-  const dim3 grid(nwg);
+  auto go = [&](auto p, auto epi) {
+    return moe::launch_rows<decltype(p)::value, decltype(epi)::value>(
+        rows_active, E, stream, q, qs, Kp, ip, sp, k_top, arow_mode, orow_mode, b, s, bi, N, G, E,
+        alpha, limit, o, out_ld, (uint8_t*)out_qs);
+  };
+  const std::integral_constant<int, 0> i0;
+  const std::integral_constant<int, 1> i1;
+  const std::integral_constant<int, 2> i2;
+  const std::integral_constant<int, 3> i3;
+  const std::integral_constant<int, 4> i4;
   if (pieces == 2 && swiglu == 2) {  // SwiGLU straight into 3 act pieces (out = their q)
     if (!out_qs || ((uintptr_t)out & 15u)) return moe::kErrUnsupported;
-    return moe::launch_gm<2, 2>(grid, lds, stream, q, qs, Kp, ip, sp, k_top, arow_mode, orow_mode,
-                                b, s, bi, N, G, E, alpha, limit, o, out_ld, xcds,
-                                (uint8_t*)out_qs);
+    return go(i2, i2);
   }
-  if (pieces == 2 && swiglu)
-    return moe::launch_gm<2, 1>(grid, lds, stream, q, qs, Kp, ip, sp, k_top, arow_mode, orow_mode,
-                                b, s, bi, N, G, E, alpha, limit, o, out_ld, xcds, nullptr);
-  if (pieces == 2)
-    return moe::launch_gm<2, 0>(grid, lds, stream, q, qs, Kp, ip, sp, k_top, arow_mode, orow_mode,
-                                b, s, bi, N, G, E, alpha, limit, o, out_ld, xcds, nullptr);
-  if (pieces == 3 && !swiglu)
-    return moe::launch_gm<3, 0>(grid, lds, stream, q, qs, Kp, ip, sp, k_top, arow_mode, orow_mode,
-                                b, s, bi, N, G, E, alpha, limit, o, out_ld, xcds, nullptr);
-  if (pieces == 4 && !swiglu)
-    return moe::launch_gm<4, 0>(grid, lds, stream, q, qs, Kp, ip, sp, k_top, arow_mode, orow_mode,
-                                b, s, bi, N, G, E, alpha, limit, o, out_ld, xcds, nullptr);
+  if (pieces == 2) return swiglu ? go(i2, i1) : go(i2, i0);
+  if (pieces == 3 && !swiglu) return go(i3, i0);
+  if (pieces == 4 && !swiglu) return go(i4, i0);
   return moe::kErrUnsupported;
 }
 

@@ -627,3 +627,27 @@ def test_mlp1_swiglu_pieces(native, block20b, n, seed):
         assert np.array_equal(a, b), np.argwhere(a != b)[:4]
     st2 = blk.forward_staged(x, pieces_epilogue=True)
     assert np.array_equal(host_bf16(st2["out"]), host_bf16(st["out"]))
+
+
+@pytest.mark.parametrize("E,H,I,n,seed,skew", [(16, 384, 192, 165, 91, False),
+                                               (16, 192, 96, 190, 92, True),
+                                               (14, 128, 96, 140, 93, False),
+                                               (13, 2880, 96, 150, 94, False)])
+def test_block_gemm_small_tile(native, E, H, I, n, seed, skew):
+    """Above 128 tokens at 40 to 48 pairs per expert on average mlp1 takes the
+    GEMM's 96-row tile (48 tokens): one, two and 23 chunks of K, one and two
+    column tiles, skewed routing (four experts of 190 tokens, four tiles with a
+    ragged last one, twelve without tokens).  Act and output against the
+    oracle."""
+    p = O.make_params(seed, num_experts=E, hidden=H, inter=I)
+    if skew:
+        p.gate_b[:] = O.f32_to_bf16(np.array([10, 9, 8, 7] + [-10] * (E - 4), np.float32))
+    x = O.make_input(seed + 100, n, hidden=H)
+    assert n > 128 and 40 * E <= 4 * n < 48 * E
+    _check_block(make_block(p), x, O.block_forward(x, p))
+
+
+def test_mlp1_swiglu_pieces_small_tile(native, block20b):
+    """The 96-row tile's act pieces = quantize_pieces of its fp32 act, bit for
+    bit, at 41 pairs per expert of the 20B shape."""
+    test_mlp1_swiglu_pieces(native, block20b, 328, 31)
