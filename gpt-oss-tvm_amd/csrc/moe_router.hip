@@ -937,7 +937,11 @@ extern "C" int moe_launch_router_logits(const void* x, const void* norm_w, const
   // experts per wave: one up to 1024 tokens (more workgroups per token
   // tile), all of them above, where 8 tokens per workgroup share each gate
   // row read (the tile's norm and t then computed once)
-  // Above 1024 tokens: 16 tokens per workgroup on the fp64 matrix cores,
+  // Above 1024 tokens, and above 40000 logits: 16 tokens per workgroup on the
+  // fp64 matrix cores (the vector form's time grows with the logits, this one's
+  // with the tokens; us, vector / matrix: E = 128 at 256, 400 and 1000 tokens 28 /
+  // 32, 41 / 34 and 86 / 55, E = 64 at 512 and 700 29 / 33 and 37 / 34, E = 32 at 1000
+  // 29 / 34),
   // epw = expert blocks of 16 per workgroup, the largest power of two up to
   // min(blocks, W) that still gives 256 workgroups (one per CU: the t tile
   // takes 96-128 KB of LDS)
@@ -945,7 +949,7 @@ extern "C" int moe_launch_router_logits(const void* x, const void* norm_w, const
     const char* v = getenv("MOE_ROUTER_MFMA_MIN");
     return v ? atoi(v) : 1024;
   }();
-  const bool mfma = n > mfma_min;
+  const bool mfma = n > mfma_min || (int64_t)n * E > 40000;
   int epw = 1;
   if (mfma) {
     const int nblk = (E + 15) / 16, gx = (n + 15) / 16;
