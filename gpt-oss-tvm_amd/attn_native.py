@@ -291,12 +291,14 @@ def qkv_gemv_rope_append(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor,
                       positions, slots, inv_freq, concentration, kv_cache, q_out, norm_w, eps)
 
 
-ROWS_MAX_TOKENS = 16
+ROWS_OUT_MAX_TOKENS, ROWS_QKV_MAX_TOKENS = 48, 64
+ROWS_NORM_MAX_TOKENS = 16   # of rows_qkv_rope_append with norm_w
+ROWS_WIDE_QKV_MAX_K = 3072  # of rows_qkv_rope_append above that
 
 
 def rows_bias_residual(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor,
                        residual: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
-    """gemv_bias_residual for at most 16 token rows."""
+    """gemv_bias_residual for at most 48 token rows."""
     return _bias_residual_fused(_lib.attn_rows_bias_residual, "attn_rows_bias_residual", x, W,
                                 bias, residual, out)
 
@@ -305,6 +307,7 @@ def rows_qkv_rope_append(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor,
                          positions: torch.Tensor, slots: torch.Tensor, inv_freq: torch.Tensor,
                          concentration: float, kv_cache: torch.Tensor, q_out: torch.Tensor,
                          norm_w: torch.Tensor | None = None, eps: float = 1e-5) -> torch.Tensor:
-    """qkv_gemv_rope_append for at most 16 token rows."""
+    """qkv_gemv_rope_append for at most 64 token rows (above 16: no norm_w, K at
+    most 3072)."""
     return _qkv_fused(_lib.attn_rows_qkv_rope_append, "attn_rows_qkv_rope_append", x, W, bias,
                       positions, slots, inv_freq, concentration, kv_cache, q_out, norm_w, eps)

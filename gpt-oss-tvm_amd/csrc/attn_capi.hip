@@ -255,8 +255,11 @@ int attn_sample_top_p(const uint16_t* logits, int64_t batch, int64_t vocab, floa
 }
 
 namespace {
-// Tokens of the fused dense projections: the GEMV and the rows entry points
-constexpr int64_t kGemvTokens = 8, kRowsTokens = 16;
+// Tokens of the fused dense projections: the GEMV entry points, the rows ones of
+// QKV and of the output.  QKV above kRowsNormTokens tokens takes them normed, and
+// rows of at most kWideQkvK.
+constexpr int64_t kGemvTokens = 8, kRowsQkvTokens = 64, kRowsOutTokens = 48;
+constexpr int64_t kRowsNormTokens = 16, kWideQkvK = 3072;
 
 int check_gemv(const void* x, int64_t M, int64_t most, int64_t K, const void* W, int64_t N,
                const void* out) {
@@ -293,6 +296,7 @@ int qkv_rope_append(int64_t most, const uint16_t* x, int64_t M, int64_t K, const
   int rc = check_gemv(x, M, most, K, W, kHeadDim * (kQHeads + 2 * kKvHeads), q_out);
   if (rc) return rc;
   if (num_pages <= 0 || num_pages > kMaxPages) return MOE_ERR_SHAPE;
+  if (M > kRowsNormTokens && (norm_w || K > kWideQkvK)) return MOE_ERR_SHAPE;
   if (!qkv_bias || !positions || !slots || !inv_freq || !kv_cache) return MOE_ERR_NULL;
   if (!a16(kv_cache) || !a4(positions) || !a4(slots) || !a4(inv_freq) ||
       ((uintptr_t)qkv_bias & 1u) || (norm_w && ((uintptr_t)norm_w & 1u)))
@@ -328,7 +332,7 @@ int attn_gemv_bias_residual(const uint16_t* x, int64_t M, int64_t K, const uint1
 int attn_rows_bias_residual(const uint16_t* x, int64_t M, int64_t K, const uint16_t* W, int64_t N,
                             const uint16_t* bias, const uint16_t* residual, uint16_t* out,
                             moe_stream_t stream) {
-  return bias_residual(kRowsTokens, x, M, K, W, N, bias, residual, out, stream);
+  return bias_residual(kRowsOutTokens, x, M, K, W, N, bias, residual, out, stream);
 }
 
 int attn_qkv_gemv_rope_append(const uint16_t* x, int64_t M, int64_t K, const uint16_t* W,
@@ -345,7 +349,7 @@ int attn_rows_qkv_rope_append(const uint16_t* x, int64_t M, int64_t K, const uin
                               const int32_t* positions, const int32_t* slots,
                               const float* inv_freq, float concentration, void* kv_cache,
                               int64_t num_pages, uint16_t* q_out, moe_stream_t stream) {
-  return qkv_rope_append(kRowsTokens, x, M, K, W, norm_w, eps, qkv_bias, positions, slots,
+  return qkv_rope_append(kRowsQkvTokens, x, M, K, W, norm_w, eps, qkv_bias, positions, slots,
                          inv_freq, concentration, kv_cache, num_pages, q_out, stream);
 }
 

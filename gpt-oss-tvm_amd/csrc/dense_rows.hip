@@ -1,4 +1,4 @@
-// Dense projections for 2 to 16 token rows on the bf16 matrix cores: the
+// Dense projections for 2 to 16 token rows (the layers' two: to 64 and 48) on the bf16 matrix cores: the
 // fused QKV nn.Linear with its bias, YaRN RoPE and the KV-cache append; the
 // attention output nn.Linear with its bias and the residual add; the
 // unembedding (model/attention.py:204,254-256; model/transformer.py:95-100).
@@ -307,6 +307,238 @@ __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// The two layer projections for 17 to 64 tokens (output: 9 to 48), NT tiles of 16.
+// Bound by the tokens' way from L2: every workgroup reads all of them (48 x 4096
+// bf16 = 393 KB against 131 KB of W for the output projection), so they stream
+// through registers beside W instead of waiting in them.  Eight waves split K; a
+// wave has its whole run of W (16 rows, QKV 32) in flight at once, the tokens two
+// chunks of kChunk steps ahead.  Loads take 64 bytes of a row with four
+// neighbouring lanes and reach the operands' order through LDS: loaded in operand
+// order, where neighbouring lanes hold different rows, a load moved about 16
+// bytes a clock (QKV with its norm 15.1, 17.0, 21.3 and 24.2 us at 17, 32, 48 and
+// 64 tokens, output 10.9, 13.5, 17.5 and 21.4; so 13.2, 13.9, 16.1 and 17.8, output
+// 8.8, 9.5, 12.0 and 15.1; at 16 tokens 7.3, rows_kernel 10.3).  Whole 128-byte lines per eight lanes changed nothing
+// (13.6, 13.8, 15.6, 20.5; output 9.3, 9.7, 11.9, 14.7).  The partial tiles, fp32
+// chains of at most 16 steps, are added over the waves in fp64 through LDS.  One
+// workgroup per CU: 180 (output) and 160 (QKV), one round.  The RMSNorm is its own
+// launch here (fused it would read the tokens twice).
+constexpr int kWideWaves = 8;
+constexpr int kWideThreads = kWideWaves * kWave;
+
+template <int NT, int EPI>
+__global__ __launch_bounds__(kWideThreads) void rows_wide_kernel(Args a) {
+#pragma clang fp contract(off)
+  constexpr int kRg = EPI == kQkv ? 2 : 1;         // row groups of the workgroup
+  constexpr int kSteps = EPI == kQkv ? 12 : 16;    // 32-wide steps of K a wave holds
+  constexpr int kChunk = EPI == kQkv ? 2 : 4;      // steps of the tokens loaded at a time
+  constexpr int kFrags = kRg + NT;                 // operand tiles of a step
+  // a wave's own: the operand tiles of two steps, then its partial result tiles
+  __shared__ __align__(16) u32x4 lds[kWideWaves][2 * kFrags][kWave];
+  static_assert(2 * kFrags >= kRg * NT, "the partial tiles take the operands' place");
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int r = lane & 15, g = lane >> 4;    // in the matrix operands and results
+  const int lr = lane >> 2, lc = lane & 3;   // in the loads: row, 16-byte chunk
+  const int M = a.M, K = a.K, N = a.N;
+  const int steps = (K + 31) / 32;
+  const int s0 = steps * wave / kWideWaves;
+  const int cnt = steps * (wave + 1) / kWideWaves - s0;
+  auto k_of = [&](int s) { return (s0 + s) * 32 + 8 * lc; };
+  auto valid = [&](int s) { return s < cnt && k_of(s) < K; };
+  auto load = [&](const uint16_t* row, int s) {
+    return *(const u32x4*)(row + min(k_of(s), K - 8));
+  };
+  const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
+  const int grp0 = blockIdx.x * kRg;
+
+  // The epilogue task of a wave: QKV: tile (wave % 2, wave / 2), both rope pairs
+  // of each lane; output: elements 2 (wave / 4) and + 1 of tile wave % 4.
+  const int trg = EPI == kQkv ? wave & 1 : 0;
+  const int tnt = EPI == kQkv ? wave >> 1 : wave & 3;
+  const int e0 = EPI == kQkv ? 0 : 2 * (wave >> 2);
+  const int tok = 16 * tnt + r;
+  const bool task = tnt < NT && tok < M;
+  const int tm = min(tok, M - 1);
+  const int erow = w_row<EPI>(grp0 + trg, 4 * g + e0);  // element 0; 1 is the next row
+  // the epilogue's operands first: the RoPE factors are taken while W streams
+  uint16_t eb[4], er[2];
+  int eslot = -1, epos = 0;
+  float ifq[2] = {0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int row = min(erow + j, N - 1);
+    eb[j] = a.bias[row];
+    if constexpr (EPI == kQkv) {
+      eb[2 + j] = a.bias[row + 32];
+      ifq[j] = a.inv_freq[row % kD];
+    } else {
+      er[j] = a.res[(size_t)tm * N + row];
+    }
+  }
+  if constexpr (EPI == kQkv) {
+    eslot = a.slots[tm];
+    epos = a.positions[tm];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  const uint16_t* xrow[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) xrow[i] = a.x + (size_t)min(16 * i + lr, M - 1) * K;
+  u32x4 xa[kChunk][NT], xb[kChunk][NT], w[kSteps][kRg];
+  auto load_x = [&](auto& dst, int s) {
+#pragma unroll
+    for (int c = 0; c < kChunk; ++c)
+#pragma unroll
+      for (int i = 0; i < NT; ++i) dst[c][i] = load(xrow[i], s + c);
+  };
+  load_x(xa, 0);
+  {
+    const uint16_t* row[kRg];
+#pragma unroll
+    for (int q = 0; q < kRg; ++q)
+      row[q] = a.W + (size_t)min(w_row<EPI>(grp0 + q, lr), N - 1) * K;
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      if (s == kChunk) load_x(xb, kChunk);
+#pragma unroll
+      for (int q = 0; q < kRg; ++q) w[s][q] = load(row[q], s);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  float cs[2] = {0.f, 0.f}, sn[2] = {0.f, 0.f};
+  if constexpr (EPI == kQkv) {
+    if (task && erow / kD < kHq + kHkv) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        double sd, cd;
+        moe::sincos_f64((double)((float)epos * ifq[j]), sd, cd);
+        cs[j] = bf2f(moe::f64_to_bf16_via_f32(cd)) * a.conc;
+        sn[j] = bf2f(moe::f64_to_bf16_via_f32(sd)) * a.conc;
+      }
+    }
+  }
+
+  f32x4 acc[kRg][NT];
+#pragma unroll
+  for (int q = 0; q < kRg; ++q)
+#pragma unroll
+    for (int i = 0; i < NT; ++i) acc[q][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // A step's tiles go through LDS from load order (lane = row, chunk) to operand
+  // order (lane = chunk, row), the chunks of a row swizzled so that the reads of
+  // 16 rows spread over the banks.  Wave-private: no barrier, program order only.
+  auto put = [&](const u32x4 (&x)[NT], int s) {
+    const bool in = valid(s);  // else zeros, in both operands
+    u32x4(*buf)[kWave] = lds[wave] + (s & 1) * kFrags;
+    const int at = lr * 4 + (lc ^ (lr >> 2));
+#pragma unroll
+    for (int q = 0; q < kRg; ++q) buf[q][at] = in ? w[s][q] : zero;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) buf[kRg + i][at] = in ? x[i] : zero;
+  };
+  u32x4 op[kFrags];
+  auto get = [&](int s) {
+    u32x4(*buf)[kWave] = lds[wave] + (s & 1) * kFrags;
+    const int at = r * 4 + (g ^ (r >> 2));
+#pragma unroll
+    for (int f = 0; f < kFrags; ++f) op[f] = buf[f][at];
+  };
+  auto products = [&]() {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int q = 0; q < kRg; ++q)
+        acc[q][i] = moe::mfma16x16x32(as_bf16x8(op[q]), as_bf16x8(op[kRg + i]), acc[q][i]);
+  };
+  auto order = [] {  // this wave's LDS accesses stay in program order
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  static_assert(kSteps % kChunk == 0 && kSteps > kChunk && kChunk > 1,
+                "two token buffers, filled in turn (the first refill follows a put)");
+  put(xa[0], 0);
+  order();
+#pragma unroll
+  for (int s = 0; s < kSteps; ++s) {
+    get(s);
+    order();
+    const int n = s + 1, c = n / kChunk;  // the next step and its chunk
+    if (n < kSteps) {
+      put(c & 1 ? xb[n % kChunk] : xa[n % kChunk], n);
+      if (n % kChunk == kChunk - 1 && (c + 2) * kChunk < kSteps)  // its last tiles are taken
+        load_x(c & 1 ? xb : xa, (c + 2) * kChunk);
+      order();
+    }
+    products();
+  }
+  f32x4(*part)[kWave] = (f32x4(*)[kWave])lds[wave];
+#pragma unroll
+  for (int q = 0; q < kRg; ++q)
+#pragma unroll
+    for (int i = 0; i < NT; ++i) part[q * NT + i][lane] = acc[q][i];
+  moe::lds_barrier();
+  if (!task) return;
+  // the waves' partials added in fp64 and rounded once
+  constexpr int kEl = EPI == kQkv ? 4 : 2;
+  double sum[kEl] = {};
+#pragma unroll
+  for (int v = 0; v < kWideWaves; ++v) {
+    const float* p = (const float*)&lds[v][trg * NT + tnt][lane] + e0;
+#pragma unroll
+    for (int i = 0; i < kEl; ++i) sum[i] += (double)p[i];
+  }
+  if constexpr (EPI == kBiasResidual) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float tb = bf2f(f2bf(bf2f(f2bf((float)sum[j])) + bf2f(eb[j])));
+      if (erow + j < N) a.out[(size_t)tok * N + erow + j] = f2bf(bf2f(er[j]) + tb);
+    }
+  } else {
+    // as rows_kernel's QKV epilogue, for the lane's two rope pairs
+    const int head = erow / kD, d = erow % kD;
+    uint16_t* dst = nullptr;
+    if (head < kHq) {
+      dst = a.q_out + ((size_t)tok * kHq + head) * kD;
+    } else if (eslot >= 0 && eslot < a.num_pages * kPage) {  // other slots are not written
+      const int kv = head < kHq + kHkv ? 0 : 1;
+      const int hk = head - kHq - kv * kHkv;
+      dst = (uint16_t*)(a.cache + (size_t)(eslot / kPage) * kPageBytes +
+                        (size_t)(kv * kHkv + hk) * kHeadBlock + (eslot % kPage) * (kD * 2));
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float lo = bf2f(f2bf(bf2f(f2bf((float)sum[j])) + bf2f(eb[j])));
+      float hi = bf2f(f2bf(bf2f(f2bf((float)sum[2 + j])) + bf2f(eb[2 + j])));
+      if (head < kHq + kHkv) {
+        const float nl = lo * cs[j] - hi * sn[j];
+        const float nh = lo * sn[j] + hi * cs[j];
+        lo = nl;
+        hi = nh;
+      }
+      if (dst) {
+        dst[d + j] = f2bf(lo);
+        dst[d + j + 32] = f2bf(hi);
+      }
+    }
+  }
+}
+
+template <int EPI>
+int launch_wide(const Args& a, unsigned grid, hipStream_t s) {
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kWideThreads), 0, s, a);
+    return hipGetLastError() == hipSuccess ? 0 : -6;
+  };
+  if constexpr (EPI == kBiasResidual)
+    if (a.M <= 16) return go(rows_wide_kernel<1, EPI>);
+  if (a.M <= 32) return go(rows_wide_kernel<2, EPI>);
+  if (a.M <= 48) return go(rows_wide_kernel<3, EPI>);
+  if constexpr (EPI == kQkv)
+    if (a.M <= 64) return go(rows_wide_kernel<4, EPI>);
+  return -6;
+}
+
 template <int EPI, bool kNorm>
 int launch(const Args& a, dim3 grid, size_t lds, hipStream_t s) {
   const bool small = a.K <= 32 * 6 * kWaves;  // 6 steps a wave; 8 cover K <= 4096
@@ -344,7 +576,7 @@ int attn_launch_rows_plain(const void* x, int M, int K, const void* W, int N, co
   return norm_w ? launch<kPlain, true>(a, grid, lds, s) : launch<kPlain, false>(a, grid, lds, s);
 }
 
-// out = bf16(res + bf16(bf16(x W^T) + bias)), M <= 16
+// out = bf16(res + bf16(bf16(x W^T) + bias)), M <= 48
 int attn_launch_rows_bias_residual(const void* x, int M, int K, const void* W, int N,
                                    const void* bias, const void* res, void* out, hipStream_t s) {
   using namespace rows;
@@ -357,10 +589,13 @@ int attn_launch_rows_bias_residual(const void* x, int M, int K, const void* W, i
   a.out = (uint16_t*)out;
   a.bias = (const uint16_t*)bias;
   a.res = (const uint16_t*)res;
-  return launch<kBiasResidual, false>(a, dim3((unsigned)(((int64_t)N + 15) / 16)), 0, s);
+  const unsigned groups = (unsigned)(((int64_t)N + 15) / 16);
+  if (M > 8) return launch_wide<kBiasResidual>(a, groups, s);
+  return launch<kBiasResidual, false>(a, dim3(groups), 0, s);
 }
 
-// the QKV projection with bias, RoPE and the cache append, M <= 16
+// the QKV projection with bias, RoPE and the cache append, M <= 64 (above 16
+// without the norm, and K <= 3072)
 int attn_launch_rows_qkv(const void* x, int M, int K, const void* W, const void* norm_w, float eps,
                          const void* bias, const int* positions, const int* slots,
                          const float* inv_freq, float conc, void* cache, int num_pages,
@@ -383,6 +618,7 @@ int attn_launch_rows_qkv(const void* x, int M, int K, const void* W, const void*
   a.num_pages = num_pages;
   a.q_out = (uint16_t*)q_out;
   const dim3 grid(a.N / 32);
+  if (M > 16) return norm_w ? -6 : launch_wide<kQkv>(a, grid.x, s);
   return norm_w ? launch<kQkv, true>(a, grid, 0, s) : launch<kQkv, false>(a, grid, 0, s);
 }
 

@@ -9,7 +9,7 @@ residual) and the alternating sliding window (even layers, attention.py:87).
 
 The dense projections round once to bf16 after fp32 accumulation, as the
 reference's matmul, and add their biases as separate bf16 ops (``nn.Linear``'s
-second op): for up to 16 tokens (decode) in hand-written kernels with the
+second op): for up to 64 (QKV) and 48 (output) tokens in hand-written kernels with the
 pre-norm, bias, RoPE and cache append (QKV) or the bias and residual (output)
 fused; for more as library GEMMs (``torch.nn.functional.linear`` without bias,
 hipBLASLt) followed by the HIP epilogue kernels.  Everything else runs in the HIP
@@ -105,17 +105,24 @@ class AttentionBlock(torch.nn.Module):
         inv_freq, self.concentration = yarn_rope_tables(config)
         self.register_buffer("inv_freq", torch.from_numpy(inv_freq).to(device), persistent=False)
 
-    def _fused(self, n: int) -> bool:
-        """Whether n tokens take the fused projections.  Between 9 and 16 tokens
-        the library's general form (any K, any weight layout) stays where the
-        fused kernels' limits do not hold.  Measured with norm and epilogues at
-        16 tokens: 20.8 + 16.0 us (QKV, output) by the library, 13.6 + 10.3
-        fused; a two-group form of the fused kernels took 15.4 us for the output
-        at 32 tokens where the library takes 13.6."""
-        if n <= A.GEMV_MAX_TOKENS or n > A.ROWS_MAX_TOKENS:
-            return n <= A.GEMV_MAX_TOKENS
-        return all(w.shape[1] <= 4096 and w.shape[1] % 8 == 0 and w.is_contiguous()
-                   and w.data_ptr() % 16 == 0 for w in (self.qkv.weight, self.out.weight))
+    def _fused(self, n: int) -> tuple[bool, bool]:
+        """Whether n tokens take the fused QKV and output projections.  From 9
+        tokens on the library's general form (any K, any weight layout) stays where
+        the fused kernels' limits do not hold.  Measured with norm and epilogues,
+        library / fused us: QKV at 16, 17, 48 and 64 tokens 19.3 / 13.4, 20.2 /
+        13.2, 21.8 / 16.1 and 24.5 / 17.8; output 14.2 / 7.3, 11.9 / 8.8, 12.8 /
+        12.0 and, past its limit of 48, 13.5 / 15.1."""
+        if n <= A.GEMV_MAX_TOKENS:
+            return True, True
+
+        def fits(w, most_k):
+            return (w.shape[1] <= most_k and w.shape[1] % 8 == 0 and w.is_contiguous()
+                    and w.data_ptr() % 16 == 0)
+
+        wide = n > A.ROWS_NORM_MAX_TOKENS
+        return (n <= A.ROWS_QKV_MAX_TOKENS
+                and fits(self.qkv.weight, A.ROWS_WIDE_QKV_MAX_K if wide else 4096),
+                n <= A.ROWS_OUT_MAX_TOKENS and fits(self.out.weight, 4096))
 
     def _window(self, tables) -> int:
         if self.sliding_window <= 0:
@@ -136,11 +143,14 @@ class AttentionBlock(torch.nn.Module):
             raise ValueError(f"{n} tokens in x, {tables.num_tokens} in the forward's tables")
         q = torch.empty((n, A.Q_HEADS, A.HEAD_DIM), dtype=x.dtype, device=x.device)
         layer = cache.layer(self.layer_idx)
-        small = self._fused(n)  # decode-sized: kernels with the norm and epilogues fused
-        if small:
-            A.rows_qkv_rope_append(x2, self.qkv.weight, self.qkv.bias, tables.positions,
+        fused_qkv, fused_out = self._fused(n)  # decode-sized: kernels with epilogues fused
+        if fused_qkv:
+            t, norm_w = x2, self.norm.weight
+            if n > A.ROWS_NORM_MAX_TOKENS:
+                t, norm_w = A.rms_norm(x2, norm_w, self.eps), None
+            A.rows_qkv_rope_append(t, self.qkv.weight, self.qkv.bias, tables.positions,
                                    tables.slots, self.inv_freq, self.concentration, layer, q,
-                                   norm_w=self.norm.weight, eps=self.eps)
+                                   norm_w=norm_w, eps=self.eps)
         else:
             t = A.rms_norm(x2, self.norm.weight, self.eps)
             qkv = F.linear(t, self.qkv.weight)
@@ -159,7 +169,7 @@ class AttentionBlock(torch.nn.Module):
                       tables.page_indices, tables.kv_len, window, self.sm_scale, self.sinks, o,
                       tables.max_kv_len)
         o2 = o.view(n, A.Q_HEADS * A.HEAD_DIM)
-        if small:
+        if fused_out:
             return A.rows_bias_residual(o2, self.out.weight, self.out.bias, x2).view(x.shape)
         y = F.linear(o2, self.out.weight)
         return A.bias_residual(x2, y, self.out.bias).view(x.shape)

@@ -139,7 +139,8 @@ MOE_API int attn_qkv_gemv_rope_append(const uint16_t* x, int64_t M, int64_t K, c
                                       float concentration, void* kv_cache, int64_t num_pages,
                                       uint16_t* q_out, moe_stream_t stream);
 
-/* The same two projections for decode batches of up to 16 tokens. */
+/* The same two projections for up to 48 (output) and 64 tokens (QKV; above 16:
+ * norm_w NULL, x normed already, K at most 3072). */
 MOE_API int attn_rows_bias_residual(const uint16_t* x, int64_t M, int64_t K, const uint16_t* W,
                                     int64_t N, const uint16_t* bias, const uint16_t* residual,
                                     uint16_t* out, moe_stream_t stream);

@@ -452,6 +452,61 @@ def test_rows_projections(A, M):
     _ulp_close(got, y, "out projection")
 
 
+@pytest.mark.parametrize("M,Kq,K,N", [(17, 2880, 4096, 2880), (32, 40, 8, 17), (33, 3072, 40, 31),
+                                      (48, 264, 2888, 16), (64, 2888, 4096, 2887)])
+def test_rows_projections_wide(A, M, Kq, K, N):
+    """The two layer projections at 17 to 64 tokens (two, three and four token
+    tiles, ragged and whole), K below, at and past whole 32-wide steps and at its
+    limit, a ragged last row group.  Sums differ from the oracle's fp64 by fp32
+    rounding only, as above."""
+    rng = np.random.default_rng(80 + M)
+    x = O.make_input(81, M, hidden=Kq)
+    W = bf(rng.standard_normal((A.QKV_DIM, Kq)) * 0.02)
+    b = bf(rng.standard_normal(A.QKV_DIM) * 0.01)
+    pos = (np.arange(M, dtype=np.int32) * 9999) % 131072
+    slots = rng.choice(4 * PAGE, M, replace=False).astype(np.int32)
+    slots[1] = 4 * PAGE                                # outside the pool: not written
+    cache = torch.zeros((4, 2, HKV, PAGE, D), dtype=torch.bfloat16, device="cuda")
+    q = torch.empty((M, HQ, D), dtype=torch.bfloat16, device="cuda")
+    inv, conc = _inv_freq_dev()
+    A.rows_qkv_rope_append(bf16_dev(x), bf16_dev(W), bf16_dev(b), i32_dev(pos), i32_dev(slots),
+                           inv, conc, cache, q)
+    rq, rk, rv = AO.split_qkv(AO.linear(x, W, b))
+    _rope_close(host_bf16(q), AO.rope(rq, pos), "q")
+    rk, c = AO.rope(rk, pos), host_bf16(cache)
+    for i in range(M):
+        if slots[i] < 4 * PAGE:
+            pg, sl = divmod(int(slots[i]), PAGE)
+            _rope_close(c[pg, 0, :, sl], rk[i], "k")
+            _ulp_close(c[pg, 1, :, sl], rv[i], "v", frac=0.03)
+            c[pg, :, :, sl] = 0
+    assert not c.any()
+    M = min(M, A.ROWS_OUT_MAX_TOKENS)
+    o = bf(np.abs(rng.standard_normal((M, K))) + 0.1)
+    Wo = bf(rng.standard_normal((N, K)) * 0.02)
+    zero, res = bf(np.zeros(N)), bf(np.zeros((M, N)))
+    args = bf16_dev(o), bf16_dev(Wo), bf16_dev(zero), bf16_dev(res)
+    _ulp_close(host_bf16(A.rows_bias_residual(*args)), AO.linear(o, Wo, None), "out projection")
+    # bias and residual: integers, so that their additions are exact after the first
+    bias, res = bf(rng.integers(-3, 4, N)), bf(rng.integers(-9, 10, (M, N)))
+    Wi, oi = bf(rng.integers(-1, 2, (N, K))), bf(np.ones((M, K)) * (np.arange(M)[:, None] % 2))
+    got = host_bf16(A.rows_bias_residual(bf16_dev(oi), bf16_dev(Wi), bf16_dev(bias), bf16_dev(res)))
+    y = AO.linear(oi, Wi, bias)
+    assert np.array_equal(got, O.f32_to_bf16(O.bf16_to_f32(res) + O.bf16_to_f32(y)))
+    # what lies past a row's end or past the last row enters no sum
+    Wo[-1, -1] = bf(np.array([np.inf]))[0]
+    y = O.bf16_to_f32(host_bf16(A.rows_bias_residual(args[0], bf16_dev(Wo), *args[2:])))
+    assert np.isinf(y[:, -1]).all() and np.isfinite(y[:, :-1]).all()
+    with pytest.raises(RuntimeError):                  # the fused norm ends at 16 tokens
+        A.rows_qkv_rope_append(bf16_dev(x), bf16_dev(W), bf16_dev(b), i32_dev(pos),
+                               i32_dev(slots), inv, conc, cache, q,
+                               norm_w=bf16_dev(bf(np.ones(Kq))))
+    big = bf16_dev(bf(np.zeros((A.ROWS_OUT_MAX_TOKENS + 1, K))))
+    with pytest.raises(RuntimeError):
+        A.rows_bias_residual(big, args[1], args[2],
+                             torch.zeros((len(big), N), dtype=torch.bfloat16, device="cuda"))
+
+
 @pytest.mark.parametrize("n,H", [(1, 8), (3, 2880), (2, 3072), (2, 3080), (2, 6144), (2, 6152)])
 def test_rms_norm_row_sizes(A, n, H):
     """Rows held in registers at both sizes, and read twice, bit for bit."""
