@@ -245,6 +245,14 @@ def test_block_internal_routing(native, E, H, I, n, seed):
     assert int(torch.count_nonzero(ws[:256])) == 0
 
 
+@pytest.mark.parametrize("E,n,seed", [(128, 313, 61), (256, 157, 62), (72, 700, 63)])
+def test_block_router_matrix_form_by_logits(native, oracle_lib, E, n, seed):
+    """Just above 40000 logits with at most 1024 tokens the router's dots move to
+    the fp64 matrix cores (ragged token tile, ragged block of experts): the same
+    bits as the oracle."""
+    test_block_internal_routing(native, E, 192, 64, n, seed)
+
+
 def test_block_workspace_reused_across_sizes(native, oracle_lib):
     """One zero-filled workspace serves calls of different sizes in turn (the
     router's arrival count sits at the workspace's start for every n and each
