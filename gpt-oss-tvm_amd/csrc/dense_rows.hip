@@ -10,7 +10,7 @@
 // 16 tokens for the price of the loads: the 201088 x 2880 unembedding at 2, 5
 // and 8 tokens 399, 750 and 1122 us on the vector ALUs, 198-201 here (5.8 TB/s);
 // QKV with its norm at 2 and 8 tokens 19.1 and 54.1 us, 12.2-12.6 here; the output
-// projection 10.6 and 34.1, 7.9-8.7 here.  (One token stays on the vector ALUs:
+// projection 10.6 and 34.1, 7.1 here (rows_wide_kernel).  (One token stays on the vector ALUs:
 // 9.1 and 6.5 us.)
 //
 // A workgroup takes 16 or 32 rows of W at a time; its sixteen waves split K
@@ -78,17 +78,16 @@ __device__ __forceinline__ int w_row(int group, int r) {
     return group * 16 + r;
 }
 
-// kSteps: 32-wide steps of K a wave holds (at most); kNorm: RMSNorm the tokens
-// first.  Row groups of a workgroup: a range walked two at a time (kPlain), two
-// (kQkv: 160 workgroups, all resident at once; with one group each the 320 ran
-// in two rounds) or one.
+// The unembedding and QKV.  kSteps: 32-wide steps of K a wave holds (at most);
+// kNorm: RMSNorm the tokens first.  Row groups of a workgroup: a range walked two
+// at a time (kPlain) or two (kQkv: 160 workgroups, all resident at once; with one
+// group each the 320 ran in two rounds).
 template <int kSteps, int EPI, bool kNorm>
 __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
 #pragma clang fp contract(off)
-  constexpr bool kTwo = EPI != kBiasResidual;  // two row groups in flight
-  constexpr int kRg = EPI == kQkv ? 2 : 1;     // row groups of a workgroup (kPlain: a range)
+  constexpr int kRg = EPI == kQkv ? 2 : 1;  // row groups of a workgroup (kPlain: a range)
   // partial tiles: of the two groups, or (kPlain) of the current and the last
-  __shared__ __align__(16) double part[kWaves][kTwo ? 2 : 1][4][kWave];
+  __shared__ __align__(16) double part[kWaves][2][4][kWave];
   __shared__ double ssq[kWaves][16];
   extern __shared__ __align__(16) uint16_t outs[];  // kPlain: [M][16 row groups of the range]
   const int t = threadIdx.x, lane = t & 63;
@@ -129,15 +128,12 @@ __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
   const int tm = min(r, M - 1);
   const int tgrp = grp0 + (EPI == kQkv ? (wave >> 1) & 1 : 0);
   const int ei = EPI == kQkv ? wave & 1 : wave & 3;
-  uint16_t eb0 = 0, eb1 = 0, er = 0;
+  uint16_t eb0 = 0, eb1 = 0;
   float ifq = 0.f, cs = 0.f, sn = 0.f;
   int eslot = -1, epos = 0, erow = 0;
-  if constexpr (EPI != kPlain) {
+  if constexpr (EPI == kQkv) {
     erow = min(w_row<EPI>(tgrp, 4 * g + ei), N - 1);
     eb0 = a.bias[erow];
-    if constexpr (EPI == kBiasResidual) er = a.res[(size_t)tm * N + erow];
-  }
-  if constexpr (EPI == kQkv) {
     eb1 = a.bias[erow + 32];
     eslot = a.slots[tm];
     epos = a.positions[tm];
@@ -149,7 +145,7 @@ __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
     for (int s = 0; s < kSteps; ++s) nw[s] = load(a.norm_w, s);
   }
   __builtin_amdgcn_sched_barrier(0);
-  u32x4 wa[kSteps], wb[kTwo ? kSteps : 1];
+  u32x4 wa[kSteps], wb[kSteps];
   auto load_w = [&](auto& dst, int group) {
     const uint16_t* row = a.W + (size_t)min(w_row<EPI>(group, r), N - 1) * K;
 #pragma unroll
@@ -157,7 +153,7 @@ __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
   };
   load_w(wa, min(grp0, grp1 - 1));
   // (behind the norm, whose weights hold registers until then)
-  if constexpr (kTwo && !kNorm) load_w(wb, min(grp0 + 1, grp1 - 1));
+  if constexpr (!kNorm) load_w(wb, min(grp0 + 1, grp1 - 1));
   __builtin_amdgcn_sched_barrier(0);
 
   if constexpr (EPI == kQkv) {  // the RoPE factors while W streams
@@ -201,7 +197,7 @@ __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
         xf[s][j] = lo | (hi << 16);
       }
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (kTwo) load_w(wb, min(grp0 + 1, grp1 - 1));
+    load_w(wb, min(grp0 + 1, grp1 - 1));
     __builtin_amdgcn_sched_barrier(0);
   }
   auto zero_tail = [&](u32x4 (&v)[kSteps]) {
@@ -268,47 +264,39 @@ __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
     zero_tail(xf);
     zero_tail(wa);
     products(wa, 0);
-    if constexpr (kTwo) {
-      zero_tail(wb);
-      products(wb, 1);
-    }
+    zero_tail(wb);
+    products(wb, 1);
     moe::lds_barrier();
     if (!task) return;
-    if constexpr (EPI == kBiasResidual) {
-      const int n = w_row<EPI>(tgrp, 4 * g + ei);
-      const float tb = bf2f(f2bf(bf2f(f2bf(total(0, ei))) + bf2f(eb0)));
-      if (n < N) a.out[(size_t)tm * N + n] = f2bf(bf2f(er) + tb);
-    } else {
-      // bias (its own bf16 rounding), then YaRN RoPE of q / k heads exactly as
-      // the standalone append kernel does, then q out or the cache slot
-      const int head = erow / kD, d = erow % kD;  // dimensions d and d + 32
-      float lo = bf2f(f2bf(bf2f(f2bf(total(tgrp - grp0, ei))) + bf2f(eb0)));
-      float hi = bf2f(f2bf(bf2f(f2bf(total(tgrp - grp0, ei + 2))) + bf2f(eb1)));
-      if (head < kHq + kHkv) {
-        const float nl = lo * cs - hi * sn;
-        const float nh = lo * sn + hi * cs;
-        lo = nl;
-        hi = nh;
-      }
-      uint16_t* dst = nullptr;
-      if (head < kHq) {
-        dst = a.q_out + ((size_t)tm * kHq + head) * kD;
-      } else if (eslot >= 0 && eslot < a.num_pages * kPage) {  // other slots are not written
-        const int kv = head < kHq + kHkv ? 0 : 1;
-        const int hk = head - kHq - kv * kHkv;
-        dst = (uint16_t*)(a.cache + (size_t)(eslot / kPage) * kPageBytes +
-                          (size_t)(kv * kHkv + hk) * kHeadBlock + (eslot % kPage) * (kD * 2));
-      }
-      if (dst) {
-        dst[d] = f2bf(lo);
-        dst[d + 32] = f2bf(hi);
-      }
+    // bias (its own bf16 rounding), then YaRN RoPE of q / k heads exactly as
+    // the standalone append kernel does, then q out or the cache slot
+    const int head = erow / kD, d = erow % kD;  // dimensions d and d + 32
+    float lo = bf2f(f2bf(bf2f(f2bf(total(tgrp - grp0, ei))) + bf2f(eb0)));
+    float hi = bf2f(f2bf(bf2f(f2bf(total(tgrp - grp0, ei + 2))) + bf2f(eb1)));
+    if (head < kHq + kHkv) {
+      const float nl = lo * cs - hi * sn;
+      const float nh = lo * sn + hi * cs;
+      lo = nl;
+      hi = nh;
+    }
+    uint16_t* dst = nullptr;
+    if (head < kHq) {
+      dst = a.q_out + ((size_t)tm * kHq + head) * kD;
+    } else if (eslot >= 0 && eslot < a.num_pages * kPage) {  // other slots are not written
+      const int kv = head < kHq + kHkv ? 0 : 1;
+      const int hk = head - kHq - kv * kHkv;
+      dst = (uint16_t*)(a.cache + (size_t)(eslot / kPage) * kPageBytes +
+                        (size_t)(kv * kHkv + hk) * kHeadBlock + (eslot % kPage) * (kD * 2));
+    }
+    if (dst) {
+      dst[d] = f2bf(lo);
+      dst[d + 32] = f2bf(hi);
     }
   }
 }
 
 // ---------------------------------------------------------------------------
-// The two layer projections for 17 to 64 tokens (output: 9 to 48), NT tiles of 16.
+// The two layer projections for 17 to 64 tokens (output: 2 to 48), NT tiles of 16.
 // Bound by the tokens' way from L2: every workgroup reads all of them (48 x 4096
 // bf16 = 393 KB against 131 KB of W for the output projection), so they stream
 // through registers beside W instead of waiting in them.  Eight waves split K; a
@@ -318,8 +306,8 @@ __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
 // order, where neighbouring lanes hold different rows, a load moved about 16
 // bytes a clock (QKV with its norm 15.1, 17.0, 21.3 and 24.2 us at 17, 32, 48 and
 // 64 tokens, output 10.9, 13.5, 17.5 and 21.4; so 13.2, 13.9, 16.1 and 17.8, output
-// 8.8, 9.5, 12.0 and 15.1; at 16 tokens 7.3, rows_kernel 10.3).  Whole 128-byte lines per eight lanes changed nothing
-// (13.6, 13.8, 15.6, 20.5; output 9.3, 9.7, 11.9, 14.7).  The partial tiles, fp32
+// 8.8, 9.5, 12.0 and 15.1; at 8 and 16 tokens 7.1 and 7.3, 8.9 and 10.3 in
+// rows_kernel's form).  Whole 128-byte lines per eight lanes changed nothing (13.6, 13.8, 15.6, 20.5; output 9.3, 9.7, 11.9, 14.7).  The partial tiles, fp32
 // chains of at most 16 steps, are added over the waves in fp64 through LDS.  One
 // workgroup per CU: 180 (output) and 160 (QKV), one round.  The RMSNorm is its own
 // launch here (fused it would read the tokens twice).
@@ -350,6 +338,9 @@ __global__ __launch_bounds__(kWideThreads) void rows_wide_kernel(Args a) {
     return *(const u32x4*)(row + min(k_of(s), K - 8));
   };
   const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
+  // one tile: sums in fp64 after every two products, as rows_kernel's
+  constexpr bool kF64 = NT == 1;
+  static_assert(!kF64 || kRg == 1, "one result tile");
   const int grp0 = blockIdx.x * kRg;
 
   // The epilogue task of a wave: QKV: tile (wave % 2, wave / 2), both rope pairs
@@ -457,6 +448,7 @@ __global__ __launch_bounds__(kWideThreads) void rows_wide_kernel(Args a) {
   };
   static_assert(kSteps % kChunk == 0 && kSteps > kChunk && kChunk > 1,
                 "two token buffers, filled in turn (the first refill follows a put)");
+  double sum64[4] = {};
   put(xa[0], 0);
   order();
 #pragma unroll
@@ -471,12 +463,23 @@ __global__ __launch_bounds__(kWideThreads) void rows_wide_kernel(Args a) {
       order();
     }
     products();
+    if constexpr (kF64)
+      if (s & 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum64[i] += (double)acc[0][0][i];
+        acc[0][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
   }
   f32x4(*part)[kWave] = (f32x4(*)[kWave])lds[wave];
+  if constexpr (kF64) {  // [element][lane]
 #pragma unroll
-  for (int q = 0; q < kRg; ++q)
+    for (int i = 0; i < 4; ++i) ((double*)part)[i * kWave + lane] = sum64[i];
+  } else {
 #pragma unroll
-    for (int i = 0; i < NT; ++i) part[q * NT + i][lane] = acc[q][i];
+    for (int q = 0; q < kRg; ++q)
+#pragma unroll
+      for (int i = 0; i < NT; ++i) part[q * NT + i][lane] = acc[q][i];
+  }
   moe::lds_barrier();
   if (!task) return;
   // the waves' partials added in fp64 and rounded once
@@ -486,7 +489,10 @@ __global__ __launch_bounds__(kWideThreads) void rows_wide_kernel(Args a) {
   for (int v = 0; v < kWideWaves; ++v) {
     const float* p = (const float*)&lds[v][trg * NT + tnt][lane] + e0;
 #pragma unroll
-    for (int i = 0; i < kEl; ++i) sum[i] += (double)p[i];
+    for (int i = 0; i < kEl; ++i) {
+      if constexpr (kF64) sum[i] += ((const double*)lds[v])[(e0 + i) * kWave + lane];
+      else sum[i] += (double)p[i];
+    }
   }
   if constexpr (EPI == kBiasResidual) {
 #pragma unroll
@@ -590,8 +596,7 @@ int attn_launch_rows_bias_residual(const void* x, int M, int K, const void* W, i
   a.bias = (const uint16_t*)bias;
   a.res = (const uint16_t*)res;
   const unsigned groups = (unsigned)(((int64_t)N + 15) / 16);
-  if (M > 8) return launch_wide<kBiasResidual>(a, groups, s);
-  return launch<kBiasResidual, false>(a, dim3(groups), 0, s);
+  return launch_wide<kBiasResidual>(a, groups, s);
 }
 
 // the QKV projection with bias, RoPE and the cache append, M <= 64 (above 16
