@@ -10,8 +10,8 @@
 // 16 tokens for the price of the loads: the 201088 x 2880 unembedding at 2, 5
 // and 8 tokens 399, 750 and 1122 us on the vector ALUs, 198-201 here (5.8 TB/s);
 // QKV with its norm at 2 and 8 tokens 19.1 and 54.1 us, 12.2-12.6 here; the output
-// projection 10.6 and 34.1, 7.1 here (rows_wide_kernel).  (One token stays on the vector ALUs:
-// 9.1 and 6.5 us.)
+// projection 10.6 and 34.1, 7.1 here (rows_wide_kernel).  (One token stays on the
+// vector ALUs: 9.1 and 6.5 us.)
 //
 // A workgroup takes 16 or 32 rows of W at a time; its sixteen waves split K
 // into contiguous runs of 32-wide steps (5 or 6 each at K = 2880), so that
