@@ -96,16 +96,27 @@ inline size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // Expert matmul dispatch (model/mlp_optimized.py:94-107 picks prefill or
 // decode kernels by token count): the tiled GEMM once the experts average 48 or
-// more pairs (each weight tile then serves many tokens), and above 128 tokens
-// (what the decode launch takes) from 40 on, where the grouped GEMV's token
-// batches overflow and it needs an encoding pass besides; the grouped GEMV below
-// that or when N is not a multiple of the GEMM's tile.  Block us, GEMV / GEMM,
-// uniform routing: 20B at 333 and 383 tokens (41.6 and 47.9 pairs per expert) 217 /
-// 202 and 215 / 205, 120B at 1500 (46.9) 1071 / 707; Zipf: 20B at 383 224 / 220, 120B
-// at 1500 904 / 782.  Lower, skewed routing loses: Zipf at 37.5 pairs 205 / 217
-// (uniform 206 / 178), 120B at 31 667 / 701 (723 / 633).
-bool use_gemm(int64_t pairs, int64_t k, int64_t E) {
-  return pairs >= 48 * E || (pairs > 128 * k && pairs >= 40 * E);
+// more pairs (each weight tile then serves many tokens); the grouped GEMV below
+// that or when N is not a multiple of the GEMM's tile.  With 64 or more experts
+// the block and its stages take the GEMM from 40 pairs on, above 128 tokens (what
+// the decode launch takes): there the GEMV's token batches overflow and it needs an
+// encoding pass besides.  Block us, GEMV / GEMM, at uniform routing and at Zipf
+// routing of beta 0.5 (the benchmark's) and 1.0:
+//   E = 64, 641 tokens (40.1 pairs)   417 / 364   412 / 391   402 / 379
+//           767 tokens (47.9)         495 / 382   446 / 409   423 / 421
+//   E = 128, 1280 tokens (40)         840 / 656   783 / 755   701 / 633
+//            1472 tokens (46)        1083 / 712   900 / 785   780 / 700
+// Fewer experts have units for a few rounds of workgroups only, and a last,
+// nearly empty round of the GEMM costs what the better tiles gain:
+//   E = 48, 528 tokens (44)           316 / 290   316 / 313   303 / 317
+//   E = 32, 328 tokens (41)           229 / 207   225 / 222   216 / 219
+//           383 tokens (47.9)         218 / 209   224 / 224   225 / 243
+//   E = 16, 168 tokens (42)           125 / 123   130 / 148   131 / 144
+// One matmul alone saves no encoding pass: moe_einsum_fused stays with 48 (E = 64,
+// 680 tokens, bf16 rows, beta 1.0: 206 / 223).
+bool tiled_matmul(int64_t pairs, int64_t E) { return pairs >= 48 * E; }
+bool tiled_block(int64_t pairs, int64_t k, int64_t E) {
+  return tiled_matmul(pairs, E) || (E >= 64 && pairs > 128 * k && pairs >= 40 * E);
 }
 
 // The decode launch combines a token's k mlp2 rows itself (the last of its k
@@ -144,9 +155,9 @@ int expert_matmul(const void* packed, int rows, int pieces, const int32_t* indpt
                   const int32_t* sorted_pairs, int k_top, int arow_mode, int orow_mode,
                   const void* blocks, const void* scales, const void* bias, int E, int N, int K,
                   int max_tokens, int pairs, int swiglu, float alpha, float limit, void* out,
-                  int out_ld, hipStream_t s) {
+                  int out_ld, bool tiled, hipStream_t s) {
   // the GEMM stores 16-byte row pieces and loads the bias 16 bytes at a time
-  if (use_gemm(pairs, k_top, E) && ((uintptr_t)out & 15u) == 0 && out_ld % 4 == 0 &&
+  if (tiled && ((uintptr_t)out & 15u) == 0 && out_ld % 4 == 0 &&
       ((uintptr_t)bias & 15u) == 0) {
     const int rc = moe_launch_mx_gemm(packed, rows, pieces, indptr, sorted_pairs, k_top,
                                       arow_mode, orow_mode, blocks, scales, bias, E, N, K, pairs,
@@ -216,16 +227,18 @@ void layout(int64_t n, int64_t E, int64_t k, int64_t H, int64_t I, size_t off[kN
 }
 
 // mlp1 + SwiGLU with act written as its three fp8 pieces (rows by sorted
-// position).  With the tiled GEMM (use_gemm) the epilogue encodes act directly (a 192-column tile holds whole
-// 32-element blocks of act): no fp32 act round trip and no encoding pass.
-// Otherwise the grouped GEMV writes fp32 act and the pieces kernel encodes it.
+// position).  With the tiled GEMM (tiled_block) the epilogue encodes act directly
+// (a 192-column tile holds whole 32-element blocks of act): no fp32 act round
+// trip and no encoding pass.  Otherwise the grouped GEMV writes fp32 act and the
+// pieces kernel encodes it.
 int mlp1_pieces(const void* t_pk, int64_t n, int64_t k, int64_t E, int64_t H, int64_t I,
                 const int32_t* indptr, const int32_t* sp, const void* blocks, const void* scales,
                 const void* bias, float alpha, float limit, float* act, void* act_pk,
                 hipStream_t s) {
   const int nk = (int)(n * k);
   int rc;
-  if (use_gemm(nk, k, E) && ((uintptr_t)bias & 15u) == 0) {
+  const bool tiled = tiled_block(nk, k, E);
+  if (tiled && ((uintptr_t)bias & 15u) == 0) {
     rc = moe_launch_mx_gemm(t_pk, (int)n, kPiecesT, indptr, sp, (int)k, 0, 1, blocks, scales,
                             bias, (int)E, (int)(2 * I), (int)H, nk, 2, alpha, limit, act_pk,
                             (int)I, (char*)act_pk + moe_pieces_q_bytes(nk, I, kPiecesAct), s);
@@ -233,7 +246,7 @@ int mlp1_pieces(const void* t_pk, int64_t n, int64_t k, int64_t E, int64_t H, in
   }
   if ((rc = expert_matmul(t_pk, (int)n, kPiecesT, indptr, sp, (int)k, 0, 1, blocks, scales, bias,
                           (int)E, (int)(2 * I), (int)H, (int)n, nk, 1, alpha, limit, act, (int)I,
-                          s)))
+                          tiled, s)))
     return rc;
   return moe_launch_pieces(act, 1, nk, (int)I, kPiecesAct, act_pk, s);
 }
@@ -357,7 +370,7 @@ int moe_einsum_fused(const void* x, int x_is_3d_f32, const int32_t* expert_indic
   if ((rc = moe_launch_pieces(x, x_is_3d_f32, rows, (int)K, pieces, packed, s))) return rc;
   return expert_matmul(packed, rows, pieces, indptr, sp, (int)k, x_is_3d_f32 ? 1 : 0, 0, blocks,
                        scales, bias, (int)E, (int)N, (int)K, (int)nk, (int)nk, 0, 0.f, 0.f, out,
-                       (int)N, s);
+                       (int)N, tiled_matmul((int64_t)nk, E), s);
 }
 
 size_t moe_pieces_bytes(int64_t rows, int64_t K, int pieces) {
@@ -388,7 +401,7 @@ int moe_mlp1_swiglu(const void* t_pieces, const int32_t* indptr, const int32_t* 
   if (!aligned16(t_pieces) || !aligned16(blocks) || ((uintptr_t)act & 3u)) return MOE_ERR_ALIGN;
   return expert_matmul(t_pieces, (int)n, kPiecesT, indptr, sorted_pairs, (int)k, 0, 1, blocks,
                        scales, bias, (int)E, (int)(2 * I), (int)H, (int)(n * k), (int)(n * k), 1,
-                       alpha, limit, act, (int)I, as_stream(stream));
+                       alpha, limit, act, (int)I, tiled_block(n * k, k, E), as_stream(stream));
 }
 
 int moe_mlp1_swiglu_pieces(const void* t_pieces, const int32_t* indptr,
@@ -419,7 +432,7 @@ int moe_mlp2(const void* act_pieces, const int32_t* indptr, const int32_t* sorte
   if (!aligned16(act_pieces) || !aligned16(blocks) || ((uintptr_t)y & 3u)) return MOE_ERR_ALIGN;
   return expert_matmul(act_pieces, (int)(n * k), kPiecesAct, indptr, sorted_pairs, (int)k, 2, 0,
                        blocks, scales, bias, (int)E, (int)H, (int)I, (int)(n * k), (int)(n * k), 0,
-                       0.f, 0.f, y, (int)H, as_stream(stream));
+                       0.f, 0.f, y, (int)H, tiled_block(n * k, k, E), as_stream(stream));
 }
 
 int moe_mlp_decode(const void* t_pieces, const int32_t* indptr, const int32_t* sorted_pairs,
@@ -527,7 +540,7 @@ static int block_forward_impl(const uint16_t* x, int64_t n, int64_t E, int64_t k
   float* logits = (float*)(ws + off[12]);
   int32_t* counts = (int32_t*)(ws + off[13]);
   int32_t* sync = (int32_t*)(ws + off[kRegionSync]);  // [E] counts, [E] status
-  const bool gemm = use_gemm(nk, k, E);
+  const bool gemm = tiled_block(nk, k, E);
   // norm, t, its pieces and the logits (and sync[0..E] = 0: the decode
   // launch's counts and status); then top-k, softmax and grouping
   void* t_qs = (char*)t_pk + moe_pieces_q_bytes(n, H, kPiecesT);
@@ -620,14 +633,14 @@ static int block_forward_impl(const uint16_t* x, int64_t n, int64_t E, int64_t k
       return rc;
   } else if ((rc = expert_matmul(t_pk, (int)n, kPiecesT, indptr, sp, (int)k, 0, 1, mlp1_blocks,
                                  mlp1_scales, mlp1_bias, (int)E, (int)(2 * I), (int)H, (int)n, nk,
-                                 1, alpha, limit, act, (int)I, s))) {
+                                 1, alpha, limit, act, (int)I, false, s))) {
     return rc;
   }
   if ((rc = mark(m, MOE_STAGE_MLP1, s))) return rc;
   if (gemm) {
     if ((rc = expert_matmul(act_pk, nk, kPiecesAct, indptr, sp, (int)k, 2, 0, mlp2_blocks,
                             mlp2_scales, mlp2_bias, (int)E, (int)H, (int)I, (int)n, nk, 0, 0.f, 0.f,
-                            y, (int)H, s)))
+                            y, (int)H, true, s)))
       return rc;
   } else if ((int64_t)nk <= 2 * E) {
     // at most two pairs per expert on average: the GEMV encodes the fp32 act

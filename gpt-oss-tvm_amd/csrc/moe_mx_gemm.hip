@@ -656,13 +656,14 @@ int launch_gm(int64_t rows_active, hipStream_t stream, const uint8_t* q, const u
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
-// Rows of a tile: 96 for two pieces (mlp1) below 48 pairs per expert on average (its
-// 48 tokens then hold most experts), else 192.  mlp1 us per launch with 96 / 192
-// rows, 20B at 333 and 383 tokens uniform 119 / 113 and 120 / 115, at 383 with Zipf
-// routing 115 / 134; 120B at 1500 uniform 405 / 407, Zipf 431 / 465.
+// Rows of a tile: 96 for mlp1 (two pieces, a SwiGLU epilogue) below 48 pairs per
+// expert on average (its 48 tokens then hold most experts), else 192.  Block us with
+// 96 / 192 rows, 128 experts at 1280, 1408 and 1535 tokens: uniform 656 / 688, 688 /
+// 701 and 720 / 713, Zipf routing of beta 0.5 755 / 768, 781 / 808 and 801 / 828, of
+// beta 1.0 633 / 646, 668 / 680 and 721 / 734.
 template <int P, int kEpi, class... A>
 int launch_rows(int64_t rows_active, int E, A... args) {
-  if constexpr (P == 2)
+  if constexpr (P == 2 && kEpi >= 1)
     if (rows_active < (int64_t)48 * E) return launch_gm<P, kEpi, 96>(rows_active, args...);
   return launch_gm<P, kEpi, 192>(rows_active, args...);
 }
