@@ -266,17 +266,19 @@ int attn_launch_gemv(const void* x, int K, const void* W, int N, void* out, cons
   a.eps = eps;
   a.bias = (const uint16_t*)bias;
   a.res = (const uint16_t*)res;
-  const size_t lds = (size_t)K * 2;
-  if (bias) {
-    constexpr int RW = 4;
-    hipLaunchKernelGGL((gemv_kernel<RW, kBiasResidual>), dim3((N + RW - 1) / RW), dim3(kThreads),
-                       lds, s, a);
-  } else {
-    constexpr int RW = 16;
-    hipLaunchKernelGGL((gemv_kernel<RW, kPlain>), dim3((N + RW - 1) / RW), dim3(kThreads), lds, s,
+  auto go = [&](auto kernel, unsigned rw) {
+    hipLaunchKernelGGL(kernel, dim3(((unsigned)N + rw - 1) / rw), dim3(kThreads), (size_t)K * 2, s,
                        a);
-  }
-  return hipGetLastError() == hipSuccess ? 0 : -6;
+    return hipGetLastError() == hipSuccess ? 0 : -6;
+  };
+  // Four rows a workgroup (58 VGPRs, eight waves per SIMD; us with
+  // 4, 8, 12 and 16 rows, 161 VGPRs and three waves: the 201088 x 2880 unembedding
+  // with its norm and the sampler behind it 201, 206, 204 and 210, alone 176, 181,
+  // 180 and 187; 131072 x 4096 177, 192, 185 and 182; 4096 x 2880 7.9, 8.8, 10.7 and
+  // 10.9).  A launch holds less than 2^32 threads: for more rows 16.
+  if (bias) return go(gemv_kernel<4, kBiasResidual>, 4);
+  constexpr int kMostGroups = (1 << 24) - 1;
+  return N <= 4 * kMostGroups ? go(gemv_kernel<4, kPlain>, 4) : go(gemv_kernel<16, kPlain>, 16);
 }
 
 int attn_launch_qkv_gemv(const void* x, int K, const void* W, const void* norm_w, float eps,

@@ -405,6 +405,24 @@ def test_gemv_several_tokens_edges(A, M, K, N):
     assert np.isinf(y[:, -1]).all() and np.isfinite(y[:, :-1]).all()
 
 
+@pytest.mark.parametrize("N", [(1 << 26) - 4, (1 << 26) - 3])
+def test_gemv_one_token_row_limits(A, N):
+    """One token over the most rows that can be launched with four a workgroup,
+    and over one more (16 a workgroup, the last one ragged): every result within
+    one bf16 ulp of the fp64 sum (eight products, fp32 rounding)."""
+    g = torch.Generator(device="cuda").manual_seed(N & 1023)
+    W = torch.randn((N, 8), generator=g, device="cuda", dtype=torch.bfloat16)
+    x = torch.rand((1, 8), generator=g, device="cuda").add_(0.1).to(torch.bfloat16)
+    got = A.gemv(x, W).view(N)
+    for part, y in zip(W.split(1 << 24), got.split(1 << 24)):
+        terms = part.double() * x[0].double()
+        ref = terms.sum(1)
+        # an ulp is at most 2^-7 of the result; the fp32 sum is off by at most
+        # eight roundings of the largest partial sum
+        bound = ref.abs() * 2.0 ** -7 + terms.abs().sum(1) * 2.0 ** -20
+        assert bool(((y.double() - ref).abs() <= bound).all())
+
+
 def _rope_close(got, ref, what):
     """As _ulp_close, for rotated pairs (d, d + 32): a projection one bf16 ulp
     off moves both results of its pair by up to an ulp of the pair's length,
