@@ -89,6 +89,7 @@ __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
   // partial tiles: of the two groups, or (kPlain) of the current and the last
   __shared__ __align__(16) double part[kWaves][2][4][kWave];
   __shared__ double ssq[kWaves][16];
+  static_assert(kSteps <= 8, "four chunks of the norm weight a step, in 32 lanes");
   extern __shared__ __align__(16) uint16_t outs[];  // kPlain: [M][16 row groups of the range]
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -139,11 +140,14 @@ __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
     epos = a.positions[tm];
     ifq = a.inv_freq[erow % kD];
   }
-  u32x4 nw[kNorm ? kSteps : 1];
-  if constexpr (kNorm) {
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) nw[s] = load(a.norm_w, s);
-  }
+  // The norm weight of the wave's K run: four chunks a step, which lane 4 s + g
+  // loads for all (16 lanes need each) and passes on through the wave's part of
+  // the partial tiles.  Held in every lane they spilled at eight steps (QKV at 2
+  // and 16 tokens, K = 4096: 23.0 and 24.9 us, 16.2 and 18.5 so; K = 3080 21.8 and
+  // 24.0, 14.4 and 16.2).
+  u32x4* const nws = (u32x4*)part[wave][0][0];
+  u32x4 nwl = u32x4{0u, 0u, 0u, 0u};
+  if constexpr (kNorm) nwl = *(const u32x4*)(a.norm_w + min(s0 * 32 + 8 * (lane & 31), K - 8));
   __builtin_amdgcn_sched_barrier(0);
   u32x4 wa[kSteps], wb[kSteps];
   auto load_w = [&](auto& dst, int group) {
@@ -180,22 +184,25 @@ __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
     ss += __shfl_xor(ss, 16, kWave);
     ss += __shfl_xor(ss, 32, kWave);
     if (g == 0) ssq[wave][r] = ss;
+    if (lane < 32) nws[lane] = nwl;
     moe::lds_barrier();
     double tot = 0.0;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) tot += ssq[w][r];
     const float rn = (float)(1.0 / sqrt(tot / (double)K + (double)a.eps));
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s)
+    for (int s = 0; s < kSteps; ++s) {
+      const u32x4 nw = nws[4 * s + g];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const uint32_t v = xf[s][j], w = nw[s][j];
+        const uint32_t v = xf[s][j], w = nw[j];
         const uint32_t lo = f2bf(__fmul_rn(__fmul_rn(__uint_as_float(v << 16), rn),
                                            __uint_as_float(w << 16)));
         const uint32_t hi = f2bf(__fmul_rn(__fmul_rn(__uint_as_float(v & 0xFFFF0000u), rn),
                                            __uint_as_float(w & 0xFFFF0000u)));
         xf[s][j] = lo | (hi << 16);
       }
+    }
     __builtin_amdgcn_sched_barrier(0);
     load_w(wb, min(grp0 + 1, grp1 - 1));
     __builtin_amdgcn_sched_barrier(0);

@@ -470,6 +470,46 @@ def test_rows_projections(A, M):
     _ulp_close(got, y, "out projection")
 
 
+@pytest.mark.parametrize("M,K,norm", [(2, 4096, True), (16, 4096, True), (3, 3080, True),
+                                      (9, 3080, False), (16, 4096, False), (13, 2888, True),
+                                      (5, 8, True), (4, 40, False)])
+def test_rows_qkv_row_sizes(A, M, K, norm):
+    """The QKV projection at 2 to 16 tokens over both register sizes (K past
+    3072 takes the larger), K below, at and past whole 32-wide steps, with the
+    norm fused and without."""
+    rng = np.random.default_rng(60 + M + K)
+    x = O.make_input(61, M, hidden=K)
+    nw = bf(rng.uniform(0.5, 1.5, K))
+    W = bf(rng.standard_normal((A.QKV_DIM, K)) * 0.02)
+    b = bf(rng.standard_normal(A.QKV_DIM) * 0.01)
+    pos = (np.arange(M, dtype=np.int32) * 9999) % 131072
+    slots = rng.choice(4 * PAGE, M, replace=False).astype(np.int32)
+    cache = torch.zeros((4, 2, HKV, PAGE, D), dtype=torch.bfloat16, device="cuda")
+    q = torch.empty((M, HQ, D), dtype=torch.bfloat16, device="cuda")
+    inv, conc = _inv_freq_dev()
+    A.rows_qkv_rope_append(bf16_dev(x), bf16_dev(W), bf16_dev(b), i32_dev(pos), i32_dev(slots),
+                           inv, conc, cache, q, norm_w=bf16_dev(nw) if norm else None)
+    rq, rk, rv = AO.split_qkv(AO.linear(O.rms_norm(x, nw, 1e-5) if norm else x, W, b))
+    _rope_close(host_bf16(q), AO.rope(rq, pos), "q")
+    c = host_bf16(cache).transpose(0, 3, 1, 2, 4).reshape(-1, 2, HKV, D)[slots]
+    _rope_close(c[:, 0], AO.rope(rk, pos), "k")
+    _ulp_close(c[:, 1], rv, "v", frac=0.03)
+
+
+@pytest.mark.parametrize("M,K,N", [(2, 8, 1), (7, 40, 17), (16, 2888, 31), (9, 4088, 48)])
+def test_rows_output_one_tile(A, M, K, N):
+    """The output projection's one-tile form (2 to 16 tokens) at ragged K and N;
+    what lies past a row's end or past the last row enters no sum."""
+    rng = np.random.default_rng(63 + K)
+    o, Wo = bf(np.abs(rng.standard_normal((M, K))) + 0.1), bf(rng.standard_normal((N, K)) * 0.02)
+    zero, res = bf16_dev(bf(np.zeros(N))), bf16_dev(bf(np.zeros((M, N))))
+    got = host_bf16(A.rows_bias_residual(bf16_dev(o), bf16_dev(Wo), zero, res))
+    _ulp_close(got, AO.linear(o, Wo, None), "out projection")
+    Wo[-1, -1] = bf(np.array([np.inf]))[0]
+    y = O.bf16_to_f32(host_bf16(A.rows_bias_residual(bf16_dev(o), bf16_dev(Wo), zero, res)))
+    assert np.isinf(y[:, -1]).all() and np.isfinite(y[:, :-1]).all()
+
+
 @pytest.mark.parametrize("M,Kq,K,N", [(17, 2880, 4096, 2880), (32, 40, 8, 17), (33, 3072, 40, 31),
                                       (48, 264, 2888, 16), (64, 2888, 4096, 2887)])
 def test_rows_projections_wide(A, M, Kq, K, N):
