@@ -25,6 +25,8 @@
 // workgroup walks a contiguous range of row groups with two groups' W in
 // flight.  The RMSNorm is the standalone kernel's arithmetic: the sum of squares
 // in fp64 from the lanes' own chunks.
+#include <stdint.h>
+
 #include "moe_common.h"
 
 namespace rows {
@@ -66,6 +68,10 @@ struct Args {
   int num_pages;
   uint16_t* q_out;
 };
+
+// Row groups of N rows of W.  In 64 bits: N may be as large as an int.
+__host__ __device__ constexpr int64_t row_groups(int N) { return ((int64_t)N + 15) / 16; }
+static_assert(row_groups(INT32_MAX) == (int64_t)1 << 27 && row_groups(16) == 1 && row_groups(17) == 2);
 
 // The W row of A row `r` of row group `group`.  QKV: eight rope pairs, a
 // pair's two dimensions in one lane's result: A rows 4 g + i hold dimensions
@@ -109,7 +115,7 @@ __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
   // this workgroup's row groups
   int grp0 = blockIdx.x * kRg, grp1 = grp0 + kRg;
   if constexpr (EPI == kPlain) {
-    const int64_t groups = (N + 15) / 16;
+    const int64_t groups = row_groups(N);
     grp0 = (int)(groups * blockIdx.x / gridDim.x);
     grp1 = (int)(groups * (blockIdx.x + 1) / gridDim.x);
   }
@@ -579,7 +585,7 @@ int attn_launch_rows_plain(const void* x, int M, int K, const void* W, int N, co
   a.norm_w = (const uint16_t*)norm_w;
   a.eps = eps;
   a.out = (uint16_t*)out;
-  const int64_t groups = ((int64_t)N + 15) / 16;
+  const int64_t groups = row_groups(N);
   // one workgroup per CU, more where a range would be longer than kMaxGroups
   const int64_t fill = groups < 256 ? groups : 256;
   const int64_t need = (groups + kMaxGroups - 1) / kMaxGroups;
@@ -602,7 +608,7 @@ int attn_launch_rows_bias_residual(const void* x, int M, int K, const void* W, i
   a.out = (uint16_t*)out;
   a.bias = (const uint16_t*)bias;
   a.res = (const uint16_t*)res;
-  const unsigned groups = (unsigned)(((int64_t)N + 15) / 16);
+  const unsigned groups = (unsigned)row_groups(N);
   return launch_wide<kBiasResidual>(a, groups, s);
 }
 
