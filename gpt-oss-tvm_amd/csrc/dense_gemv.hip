@@ -131,7 +131,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(Args a) {
 #pragma unroll
     for (int i = 0; i < RW; ++i)
       wv[it][i] = *(const u32x4*)(a.W + (size_t)min(rows[i], N - 1) * K + cc * 8);
-    nwv[it] = *(const u32x4*)(nw + cc * 8);
+    nwv[it] = *(const moe::u32x4_any*)(nw + cc * 8);  // (a caller's slice at any element)
   }
   __builtin_amdgcn_sched_barrier(0);
   // the RoPE factors while W streams

@@ -153,7 +153,8 @@ __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
   // 24.0, 14.4 and 16.2).
   u32x4* const nws = (u32x4*)part[wave][0][0];
   u32x4 nwl = u32x4{0u, 0u, 0u, 0u};
-  if constexpr (kNorm) nwl = *(const u32x4*)(a.norm_w + min(s0 * 32 + 8 * (lane & 31), K - 8));
+  if constexpr (kNorm)  // (a caller's slice at any element)
+    nwl = *(const moe::u32x4_any*)(a.norm_w + min(s0 * 32 + 8 * (lane & 31), K - 8));
   __builtin_amdgcn_sched_barrier(0);
   u32x4 wa[kSteps], wb[kSteps];
   auto load_w = [&](auto& dst, int group) {

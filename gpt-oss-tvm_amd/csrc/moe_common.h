@@ -10,6 +10,9 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+// The same where only the elements' alignment is given: still one 16-byte load
+// (the hardware takes any address), without a promise that does not hold.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
 
 constexpr int kWave = 64;
 

@@ -115,8 +115,8 @@ MOE_API int attn_embedding(const int32_t* ids, int64_t n, const uint16_t* table,
 /* Decode-sized dense projection (nn.Linear's matmul for M <= 8 tokens):
  * out[m][n] = bf16(sum_k t[m][k] W[n][k]), fp32 accumulation, one bf16
  * rounding, where t = x, or t = RMSNorm(x) with weight norm_w and eps when
- * norm_w is not NULL (the same arithmetic as attn_rms_norm).  x [M, K], W [N,
- * K], out [M, N] bf16; K % 8 == 0, K <= 4096.  Replaces the final norm and
+ * norm_w is not NULL (the same arithmetic as attn_rms_norm; norm_w [K] may
+ * begin at any element).  x [M, K], W [N, K], out [M, N] bf16; K % 8 == 0, K <= 4096.  Replaces the final norm and
  * the unembedding nn.Linear at decode (model/transformer.py:63,95-100). */
 MOE_API int attn_gemv(const uint16_t* x, int64_t M, int64_t K, const uint16_t* W, int64_t N,
                       const uint16_t* norm_w, float eps, uint16_t* out, moe_stream_t stream);

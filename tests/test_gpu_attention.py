@@ -496,6 +496,31 @@ def test_rows_qkv_row_sizes(A, M, K, norm):
     _ulp_close(c[:, 1], rv, "v", frac=0.03)
 
 
+@pytest.mark.parametrize("M", [1, 2, 8])
+def test_norm_weight_at_any_element(A, M):
+    """The norm weight may be a slice that starts at any element: the same bits
+    as from a copy of its own, in the unembedding and in QKV."""
+    rng = np.random.default_rng(65 + M)
+    K, N = 2880, 96
+    x, W, Wq = (bf16_dev(bf(rng.standard_normal(s) * 0.1)) for s in ((M, K), (N, K), (A.QKV_DIM, K)))
+    b = bf16_dev(bf(rng.standard_normal(A.QKV_DIM) * 0.01))
+    pos = torch.arange(M, dtype=torch.int32, device="cuda")
+    inv, conc = _inv_freq_dev()
+    held = bf16_dev(bf(rng.uniform(0.5, 1.5, K + 8)))
+
+    def both(nw):
+        cache = torch.zeros((1, 2, HKV, PAGE, D), dtype=torch.bfloat16, device="cuda")
+        q = torch.empty((M, HQ, D), dtype=torch.bfloat16, device="cuda")
+        A.rows_qkv_rope_append(x, Wq, b, pos, pos, inv, conc, cache, q, norm_w=nw)
+        return A.gemv(x, W, norm_w=nw), q, cache
+
+    for first in (1, 2, 5):
+        nw = held[first:first + K]
+        assert nw.data_ptr() % 16
+        for got, want in zip(both(nw), both(nw.clone())):
+            assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("M,K,N", [(2, 8, 1), (7, 40, 17), (16, 2888, 31), (9, 4088, 48)])
 def test_rows_output_one_tile(A, M, K, N):
     """The output projection's one-tile form (2 to 16 tokens) at ragged K and N;
