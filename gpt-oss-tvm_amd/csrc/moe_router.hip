@@ -248,7 +248,7 @@ __global__ __launch_bounds__(64 * W) void moe_router_kernel(
 // Router logits: workgroup (bx, by) of W waves computes the logits of tokens
 // [TT bx, TT bx + TT) for experts [W epw by, W epw (by + 1)): wave w takes
 // experts W (epw by + i) + w, i < epw, one after another (the next gate row
-// loads while the current one's dots run).  Up to 1024 tokens epw = 1: the
+// loads while the current one's dots run).  In the vector form epw = 1: the
 // experts spread over several workgroups per token.
 //  1  the threads load the token rows and the norm weight cooperatively (one
 //     16-byte chunk per thread and token); each wave loads its gate row;
@@ -918,10 +918,26 @@ extern "C" int moe_launch_router(const void* x, const void* norm_w, const void* 
                                   w_out, nullptr, nullptr, stream);
 }
 
+namespace {
+// Whether the logits are taken by the fp64 matrix cores, 16 tokens per workgroup:
+// above 1024 tokens, and above 40000 logits (the vector form's time grows with the
+// logits, this one's with the tokens; us, vector / matrix: E = 128 at 256, 400 and
+// 1000 tokens 28 / 32, 41 / 34 and 86 / 55, E = 64 at 512 and 700 29 / 33 and 37 /
+// 34, E = 32 at 1000 29 / 34).  MOE_ROUTER_MFMA_MIN, where it is set, takes the
+// place of both lines (tuning runs): the matrix form above that many tokens.
+constexpr bool router_matrix_form(int64_t n, int64_t E, bool set, int64_t over) {
+  return set ? n > over : n > 1024 || n * E > 40000;
+}
+static_assert(router_matrix_form(313, 128, false, 0) && !router_matrix_form(312, 128, false, 0) &&
+              router_matrix_form(1025, 32, false, 0) && !router_matrix_form(1024, 32, false, 0));
+static_assert(!router_matrix_form(1000, 128, true, 2000) && router_matrix_form(2001, 8, true, 2000) &&
+              router_matrix_form(1, 8, true, 0));
+}  // namespace
+
 // Logits of the n tokens into logits[n][E] (fp32 holding bf16 values), t,
-// and (pq != null, H % 32 == 0) the two fp8 pieces of t.  One expert per
-// wave (n <= 1024) or all E per workgroup; TT tokens per workgroup share each
-// gate row read.  zero_e (if not null): E + 1 ints set to zero by workgroup
+// and (pq != null, H % 32 == 0) the two fp8 pieces of t.  One expert per wave,
+// or (router_matrix_form) blocks of 16 on the matrix cores; TT tokens per
+// workgroup share each gate row read.  zero_e (if not null): E + 1 ints set to zero by workgroup
 // (0, 0) (the decode launch's completion counts and its status word).
 extern "C" int moe_launch_router_logits(const void* x, const void* norm_w, const void* gate_w,
                                         const void* gate_b, int n, int H, int E, float eps,
@@ -934,22 +950,18 @@ extern "C" int moe_launch_router_logits(const void* x, const void* norm_w, const
   uint16_t* pt = (uint16_t*)t_out;
   uint8_t *q = (uint8_t*)pq, *qs = (uint8_t*)pqs;
   constexpr int W = 8;
-  // experts per wave: one up to 1024 tokens (more workgroups per token
-  // tile), all of them above, where 8 tokens per workgroup share each gate
-  // row read (the tile's norm and t then computed once)
-  // Above 1024 tokens, and above 40000 logits: 16 tokens per workgroup on the
-  // fp64 matrix cores (the vector form's time grows with the logits, this one's
-  // with the tokens; us, vector / matrix: E = 128 at 256, 400 and 1000 tokens 28 /
-  // 32, 41 / 34 and 86 / 55, E = 64 at 512 and 700 29 / 33 and 37 / 34, E = 32 at 1000
-  // 29 / 34),
-  // epw = expert blocks of 16 per workgroup, the largest power of two up to
-  // min(blocks, W) that still gives 256 workgroups (one per CU: the t tile
-  // takes 96-128 KB of LDS)
-  static const int mfma_min = [] {  // MOE_ROUTER_MFMA_MIN overrides (tuning runs)
+  // Vector form: one expert per wave.  Matrix form: epw = expert blocks of 16 per
+  // workgroup, the largest power of two up to min(blocks, W) that still gives 256
+  // workgroups (one per CU: the t tile takes 96-128 KB of LDS).
+  struct Line {
+    bool set;
+    int over;
+  };
+  static const Line line = [] {
     const char* v = getenv("MOE_ROUTER_MFMA_MIN");
-    return v ? atoi(v) : 1024;
+    return Line{v != nullptr, v ? atoi(v) : 0};
   }();
-  const bool mfma = n > mfma_min || (int64_t)n * E > 40000;
+  const bool mfma = router_matrix_form(n, E, line.set, line.over);
   int epw = 1;
   if (mfma) {
     const int nblk = (E + 15) / 16, gx = (n + 15) / 16;
