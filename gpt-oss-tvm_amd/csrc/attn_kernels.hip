@@ -133,83 +133,74 @@ __global__ __launch_bounds__(kRmsThreads) void rms_norm_kernel(const u32x4* __re
 // cos/sin of fp32(position) * inv_freq are evaluated in fp64, rounded to fp32
 // and then to bf16 (the rope's .astype(dtype)), then scaled by the fp32
 // concentration; the rotation rounds each product and the difference / sum
-// separately (no contraction).  A workgroup takes kRopeTok tokens; their 32
-// cos/sin pairs each are taken once, for all 72 heads, into LDS (one pair per
-// thread and (head, d) before: bound by the fp64 sine and cosine, 52 us at
-// 4096 tokens against 14.6 now, 5.8 TB/s of its 84 MB in and out), while
-// the first token's loads are in flight.  One thread per eight rotation pairs
-// (d .. d + 7, + 32) of a head: 16-byte loads and stores.
+// separately (no contraction).  A workgroup takes one token; its 32 cos/sin pairs
+// are taken once, for all 72 heads, into LDS (one pair per thread and (head, d)
+// before: bound by the fp64 sine and cosine, 52 us at 4096 tokens against 15.7
+// now, 5.3 TB/s of its 84 MB in and out), while the token's loads are in flight.
+// One thread per eight rotation pairs (d .. d + 7, + 32) of a head: 16-byte loads
+// and stores.  (Four tokens a workgroup gained nothing: 2048, 4096, 6144 and 8192
+// tokens 10.0 -> 11.4, 18.8 -> 20.3, 25.0 -> 27.4 and 31.8 -> 33.2 us with qkv from
+// HBM, 4096 and 8192 from the cache 15.7 -> 15.5 and 26.6 -> 28.6.)
 constexpr int kRopeThreads = kQkvHeads * 4;  // 320: (head, quarter of its 32 pairs)
+constexpr int kRopeRow = 1 << 20;            // workgroups of a grid row
 
-template <int kRopeTok>
 __global__ __launch_bounds__(kRopeThreads) void qkv_rope_append_kernel(
     const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ bias, int n,
     const int* __restrict__ positions, const int* __restrict__ slots,
     const float* __restrict__ inv_freq, float conc, uint8_t* __restrict__ cache, int num_pages,
     uint16_t* __restrict__ q_out) {
 #pragma clang fp contract(off)
-  __shared__ float cs[kRopeTok][32], sn[kRopeTok][32];
+  __shared__ float cs[32], sn[32];
   const int t = threadIdx.x;
-  const int tok0 = blockIdx.x * kRopeTok, ntok = min(kRopeTok, n - tok0);
+  const int tok = blockIdx.x + blockIdx.y * kRopeRow;
+  if (tok >= n) return;
   const int head = t >> 2, d = (t & 3) * 8;
   const size_t col = (size_t)head * kD + d;
-  u32x4 lo[kRopeTok], hi[kRopeTok];
-  int slot[kRopeTok];
-#pragma unroll
-  for (int j = 0; j < kRopeTok; ++j) {
-    const int tok = tok0 + min(j, ntok - 1);
-    const uint16_t* src = qkv + (size_t)tok * (kQkvHeads * kD) + col;
-    lo[j] = *(const u32x4*)src;
-    hi[j] = *(const u32x4*)(src + 32);
-    slot[j] = slots[tok];
-  }
+  const uint16_t* src = qkv + (size_t)tok * (kQkvHeads * kD) + col;
+  const u32x4 lo = *(const u32x4*)src, hi = *(const u32x4*)(src + 32);
+  const int slot = slots[tok];
   const u32x4 blo = *(const u32x4*)(bias + col), bhi = *(const u32x4*)(bias + col + 32);
-  if (t < 32 * kRopeTok) {
-    const int j = t >> 5;
-    const float freq = (float)positions[tok0 + min(j, ntok - 1)] * inv_freq[t & 31];
+  if (t < 32) {
+    const float freq = (float)positions[tok] * inv_freq[t];
     double s, c;
     moe::sincos_f64((double)freq, s, c);
-    cs[j][t & 31] = bf2f(moe::f64_to_bf16_via_f32(c)) * conc;
-    sn[j][t & 31] = bf2f(moe::f64_to_bf16_via_f32(s)) * conc;
+    cs[t] = bf2f(moe::f64_to_bf16_via_f32(c)) * conc;
+    sn[t] = bf2f(moe::f64_to_bf16_via_f32(s)) * conc;
   }
   moe::lds_barrier();
+  u32x4 olo, ohi;
 #pragma unroll
-  for (int j = 0; j < kRopeTok; ++j) {
-    if (j >= ntok) break;
-    u32x4 olo, ohi;
+  for (int i = 0; i < 4; ++i) {
+    uint32_t wl = 0, wh = 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      uint32_t wl = 0, wh = 0;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {  // the word's two dimensions
-        auto val = [&](uint32_t w) { return __uint_as_float(h ? w & 0xFFFF0000u : w << 16); };
-        float l = bf2f(f2bf(val(lo[j][i]) + val(blo[i])));
-        float u = bf2f(f2bf(val(hi[j][i]) + val(bhi[i])));
-        if (head < kHq + kHkv) {
-          const float c = cs[j][d + 2 * i + h], s = sn[j][d + 2 * i + h];
-          const float nl = l * c - u * s;
-          const float nu = l * s + u * c;
-          l = nl;
-          u = nu;
-        }
-        wl |= (uint32_t)f2bf(l) << (16 * h);
-        wh |= (uint32_t)f2bf(u) << (16 * h);
+    for (int h = 0; h < 2; ++h) {  // the word's two dimensions
+      auto val = [&](uint32_t w) { return __uint_as_float(h ? w & 0xFFFF0000u : w << 16); };
+      float l = bf2f(f2bf(val(lo[i]) + val(blo[i])));
+      float u = bf2f(f2bf(val(hi[i]) + val(bhi[i])));
+      if (head < kHq + kHkv) {
+        const float c = cs[d + 2 * i + h], s = sn[d + 2 * i + h];
+        const float nl = l * c - u * s;
+        const float nu = l * s + u * c;
+        l = nl;
+        u = nu;
       }
-      olo[i] = wl;
-      ohi[i] = wh;
+      wl |= (uint32_t)f2bf(l) << (16 * h);
+      wh |= (uint32_t)f2bf(u) << (16 * h);
     }
-    uint16_t* dst = nullptr;
-    if (head < kHq) {
-      dst = q_out + ((size_t)(tok0 + j) * kHq + head) * kD;
-    } else if (slot[j] >= 0 && slot[j] < num_pages * kPage) {  // other slots are not written
-      const int kv = head < kHq + kHkv ? 0 : 1;
-      const int hk = head - kHq - kv * kHkv;
-      dst = (uint16_t*)kv_row(cache, slot[j] / kPage, kv, hk, slot[j] % kPage);
-    }
-    if (dst) {
-      *(u32x4*)(dst + d) = olo;
-      *(u32x4*)(dst + d + 32) = ohi;
-    }
+    olo[i] = wl;
+    ohi[i] = wh;
+  }
+  uint16_t* dst = nullptr;
+  if (head < kHq) {
+    dst = q_out + ((size_t)tok * kHq + head) * kD;
+  } else if (slot >= 0 && slot < num_pages * kPage) {  // other slots are not written
+    const int kv = head < kHq + kHkv ? 0 : 1;
+    const int hk = head - kHq - kv * kHkv;
+    dst = (uint16_t*)kv_row(cache, slot / kPage, kv, hk, slot % kPage);
+  }
+  if (dst) {
+    *(u32x4*)(dst + d) = olo;
+    *(u32x4*)(dst + d + 32) = ohi;
   }
 }
 
@@ -1015,15 +1006,13 @@ int attn_launch_rms_norm(const void* x, int n, int H, const void* w, float eps, 
 int attn_launch_qkv_rope_append(const void* qkv, const void* bias, int n, const int* positions,
                                 const int* slots, const float* inv_freq, float conc, void* cache,
                                 int num_pages, void* q_out, hipStream_t s) {
-  // several tokens a workgroup once there are workgroups enough without
-  auto go = [&](auto kernel, int per) {
-    hipLaunchKernelGGL(kernel, dim3((n + per - 1) / per), dim3(attn::kRopeThreads), 0, s,
-                       (const uint16_t*)qkv, (const uint16_t*)bias, n, positions, slots, inv_freq,
-                       conc, (uint8_t*)cache, num_pages, (uint16_t*)q_out);
-    return hipGetLastError() == hipSuccess ? 0 : -6;
-  };
-  return n >= 4096 ? go(attn::qkv_rope_append_kernel<4>, 4)
-                   : go(attn::qkv_rope_append_kernel<1>, 1);
+  // (2^24 tokens: in rows, as a launch holds less than 2^32 threads in each)
+  const int rows = (n + attn::kRopeRow - 1) / attn::kRopeRow;
+  hipLaunchKernelGGL(attn::qkv_rope_append_kernel, dim3(rows > 1 ? attn::kRopeRow : n, rows),
+                     dim3(attn::kRopeThreads), 0, s, (const uint16_t*)qkv, (const uint16_t*)bias, n,
+                     positions, slots, inv_freq, conc, (uint8_t*)cache, num_pages,
+                     (uint16_t*)q_out);
+  return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 
 int attn_launch_decode(const void* q, int batch, const void* cache, const int* page_indptr,

@@ -601,8 +601,7 @@ def test_rms_norm_row_sizes(A, n, H):
 
 @pytest.mark.parametrize("n", [4096, 4099])
 def test_qkv_rope_append_many_tokens(A, n):
-    """Four tokens a workgroup, with and without a ragged last one, at positions
-    over the whole context, bit for bit."""
+    """Long prompts, at positions over the whole context, bit for bit."""
     rng = np.random.default_rng(n)
     qkv = bf(rng.standard_normal((n, A.QKV_DIM)))
     bias = bf(rng.standard_normal(A.QKV_DIM) * 0.1)
@@ -619,6 +618,31 @@ def test_qkv_rope_append_many_tokens(A, n):
     c = host_bf16(cache).transpose(0, 3, 1, 2, 4).reshape(-1, 2, HKV, D)
     np.testing.assert_array_equal(c[slots, 0], AO.rope(rk, pos))
     np.testing.assert_array_equal(c[slots, 1], rv)
+
+
+def test_qkv_rope_append_rows_of_workgroups(A):
+    """More tokens than a grid row's workgroups: the last of the first row and
+    those of the second as in a call of their own."""
+    n = (1 << 20) + 3
+    g = torch.Generator(device="cuda").manual_seed(5)
+    few = torch.randn((6, A.QKV_DIM), generator=g, device="cuda").to(torch.bfloat16)
+    bias = torch.randn(A.QKV_DIM, generator=g, device="cuda").to(torch.bfloat16)
+    inv, conc = _inv_freq_dev()
+
+    def run(qkv, pos, slots):
+        cache = torch.zeros((1, 2, HKV, PAGE, D), dtype=torch.bfloat16, device="cuda")
+        q = torch.empty((len(qkv), HQ, D), dtype=torch.bfloat16, device="cuda")
+        A.qkv_rope_append(qkv, bias, pos, slots, inv, conc, cache, q)
+        return q, cache
+
+    pos6, slots6 = i32_dev(np.arange(6) * 21001), i32_dev(np.array([4, 1, 15, 0, 9, 7]))
+    want_q, want_cache = run(few, pos6, slots6)
+    qkv = torch.zeros((n, A.QKV_DIM), dtype=torch.bfloat16, device="cuda")
+    pos = torch.zeros(n, dtype=torch.int32, device="cuda")
+    slots = torch.full((n,), -1, dtype=torch.int32, device="cuda")
+    qkv[n - 6:], pos[n - 6:], slots[n - 6:] = few, pos6, slots6
+    q, cache = run(qkv, pos, slots)
+    assert torch.equal(q[n - 6:], want_q) and torch.equal(cache, want_cache)
 
 
 @pytest.mark.parametrize("qlens,prefix,bound", [
