@@ -138,7 +138,8 @@ def prefill(q: torch.Tensor, q_indptr: torch.Tensor, max_q_len: int, kv_cache: t
 
     ``max_kv_len`` (0: unknown) bounds kv_len; with it, calls of few query tiles
     over many keys share the keys out over more workgroups (their partial
-    results in a buffer allocated for the call)."""
+    results in a buffer allocated for the call).  How many follows from the whole
+    call: a sequence's last bits may change with its neighbours and the bound."""
     _expect(q, "q", torch.bfloat16)
     n = q.shape[0]
     _expect(q, "q", torch.bfloat16, (n, Q_HEADS, HEAD_DIM))

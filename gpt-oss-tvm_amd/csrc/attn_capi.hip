@@ -79,9 +79,14 @@ int64_t decode_splits(int64_t batch, int64_t max_span) {
 // Measured, us without and with (new tokens + cached): 9 + 1500 60.6 and 18.3, 64 +
 // 8000 296 and 37.7, 300 + 600 43.3 and 31.4, 300 + 6000 238 and 86, 1024 + 0 46.3 and
 // 45.2.  One round more than fits cost more than the shares gained (300 + 6000 in
-// 560 workgroups 104 us); 700 + 0 in two shares took 35.3 against 33.3.
+// 560 workgroups 104 us); 700 + 0 in two shares took 35.3 against 33.3.  The shares
+// follow from the whole call, so a sequence's last bits depend on what else is in
+// it (decode's do not); merged in fp32, they are no further off than the plain
+// form (against 64 bits, plain and shared: 9 + 1500 1.35e-4 and 1.11e-4, 300 + 6000
+// 1.35e-4 and 1.28e-4, 1024 + 0 1.14e-4 and 1.08e-4).
 constexpr int64_t kPfSplitKeys = 192, kPfMaxSplits = 16, kPfWorkgroups = 512;
 int64_t prefill_splits(int64_t batch, int64_t max_q_len, int64_t max_kv_len, int64_t window) {
+  if (batch <= 0 || batch > kPfWorkgroups) return 1;  // (and no overflow below)
   const int64_t wgs = (max_q_len + 63) / 64 * batch * 16;
   const int64_t keys = (window > 0 ? std::min(max_kv_len, window + 64) : max_kv_len) - max_q_len / 2;
   if (wgs <= 0) return 1;

@@ -89,7 +89,10 @@ MOE_API int attn_prefill(const uint16_t* q, const int32_t* q_indptr, int64_t bat
 /* attn_prefill for calls whose query tiles would not fill the chip (a short text
  * over a long cached prefix): each tile's keys are shared out over several
  * workgroups, whose partial results wait in `workspace` (q has `rows` rows, max_kv_len
- * bounds kv_len and only chooses the split).  attn_prefill_workspace_bytes is 0
+ * bounds kv_len and only chooses the split).  The split follows from batch,
+ * max_q_len, max_kv_len and window: a sequence's result is the same for any
+ * split up to fp32 rounding, but its last bits may change with the other
+ * sequences of the call and with the bound.  attn_prefill_workspace_bytes is 0
  * where the plain form is taken; the workspace needs no initialisation. */
 MOE_API size_t attn_prefill_workspace_bytes(int64_t rows, int64_t batch, int64_t max_q_len,
                                             int64_t max_kv_len, int32_t window);

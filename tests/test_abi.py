@@ -82,6 +82,20 @@ def test_attention_validation(native):
     assert lib.attn_bias_residual(p, p, p, 2, 2882, p, None) == codes["MOE_ERR_SHAPE"]
 
 
+def test_prefill_workspace_bytes(native):
+    """Shares only where a call's query tiles leave the chip idle, for any
+    argument: a batch beyond 64 bits of workgroups has none."""
+    import attn_native  # noqa: F401  (registers the signatures)
+    need = native.lib().attn_prefill_workspace_bytes
+    assert need(300, 1, 300, 6300, 0) == 6 * 300 * 64 * 66 * 4   # 5 tiles: 512 / 80 workgroups
+    assert need(4096, 1, 4096, 4096, 0) == 0                     # tiles enough
+    assert need(300, 1, 300, 0, 0) == 0                          # no bound given
+    assert need(64, 1, 64, 8064, 128) == 0                       # a short window
+    assert need(64, 1, 64, 8064, 1000) == 5 * 64 * 64 * 66 * 4   # 1032 keys
+    for batch in (-1, 0, 33, 513, (1 << 60) + 1, (1 << 62) + 3, (1 << 63) - 1):
+        assert need(300, batch, 300, 6300, 0) == 0, batch
+
+
 def test_internal_launchers_are_hidden(native):
     with pytest.raises(AttributeError):
         getattr(native.lib(), "moe_launch_mx_gemv")

@@ -671,3 +671,26 @@ def test_prefill_attention_shared_keys(A, qlens, prefix, bound):
         rows = slice(q_indptr[b], q_indptr[b + 1])
         o, lse = AO.attention(q[rows], seqs.k[b], seqs.v[b], np.arange(L - ql, L), 0)
         close(got[rows], AO.sink_scale(o, lse, sinks))
+
+
+@pytest.mark.parametrize("window,qlens,prefix", [(352, [9], [1500]), (1000, [64, 1, 130], [3000, 40, 990]),
+                                                 (1500, [300], [4001])])
+def test_prefill_attention_shared_keys_window(A, window, qlens, prefix):
+    """Sliding windows wide enough to be shared out: the shares begin at the
+    first key that the tile's first row sees."""
+    lengths = [p + q for p, q in zip(prefix, qlens)]
+    n = sum(qlens)
+    assert A._lib.attn_prefill_workspace_bytes(n, len(qlens), max(qlens), max(lengths), window) > 0
+    seqs = PagedSeqs(93 + n, lengths)
+    rng = np.random.default_rng(94 + n)
+    q = bf(2.0 * rng.standard_normal((n, HQ, D)))
+    sinks = bf(rng.standard_normal(HQ))
+    q_indptr = np.concatenate([[0], np.cumsum(qlens)]).astype(np.int32)
+    out = torch.empty((n, HQ, D), dtype=torch.bfloat16, device="cuda")
+    A.prefill(bf16_dev(q), i32_dev(q_indptr), max(qlens), seqs.cache, seqs.page_indptr,
+              seqs.page_indices, seqs.kv_len, window, SCALE, bf16_dev(sinks), out, max(lengths))
+    got = host_bf16(out)
+    for b, (L, ql) in enumerate(zip(lengths, qlens)):
+        rows = slice(q_indptr[b], q_indptr[b + 1])
+        o, lse = AO.attention(q[rows], seqs.k[b], seqs.v[b], np.arange(L - ql, L), window)
+        close(got[rows], AO.sink_scale(o, lse, sinks))
