@@ -328,6 +328,115 @@ def test_attention_block_prefill_then_decode(A, layer_idx):
     assert cache.seq_len(0) == n0 + 3
 
 
+# tokens of a forward -> (fused QKV, fused output) at gpt-oss shapes
+_ROUTES = {2: (True, True), 8: (True, True), 9: (True, True), 16: (True, True), 17: (True, True),
+           48: (True, True), 49: (True, False), 64: (True, False), 65: (False, False)}
+
+
+@pytest.fixture(scope="module")
+def attn_block(A):
+    p = AO.make_attn_params(57)
+    return p, _block(A, p, 1)
+
+
+def _held(cache, layer, tables):
+    """Keys and values [L, 8, 64] (bf16 bits) of each sequence of a forward."""
+    data, ptr = host_bf16(cache.data[layer]), tables.page_indptr.cpu().numpy()
+    pages, lens = tables.page_indices.cpu().numpy(), tables.kv_len.cpu().numpy()
+    kv = [data[pages[a:b]].transpose(1, 0, 3, 2, 4).reshape(2, -1, HKV, D)
+          for a, b in zip(ptr, ptr[1:])]
+    return [(c[0, :L], c[1, :L]) for c, L in zip(kv, lens)]
+
+
+@pytest.mark.parametrize("n", sorted(_ROUTES))
+def test_attention_block_routes_decode(A, attn_block, n):
+    """A decode batch of n sequences, on both sides of every line between the
+    fused projections and the library's: the norm in the projection up to 16
+    tokens, on its own above, output by the library above 48, QKV above 64."""
+    from model.kv_cache import PagedKVCache
+    p, blk = attn_block
+    assert blk._fused(n) == _ROUTES[n]
+    rng = np.random.default_rng(n)
+    lengths = rng.integers(0, 70, n)
+    lengths[0] = 0                                        # a first token
+    cache = PagedKVCache(num_layers=2, num_pages=6 * n, max_batch=n, max_tokens=80 * n)
+    cache.data[1].copy_(bf16_dev(bf(rng.standard_normal(tuple(cache.data[1].shape)))))
+    for i in range(n):
+        cache.add_sequence(i)
+        cache.enable_sliding_window(i, 128)
+        if lengths[i]:
+            cache.begin_forward([i], [lengths[i]])
+            cache.end_forward()
+    x = O.make_input(58, n)
+    tables = cache.begin_forward(list(range(n)), [1] * n)
+    before = _held(cache, 1, tables)
+    got = host_bf16(blk(bf16_dev(x).view(n, 1, 2880), cache).view(n, 2880))
+    q, k, v = AO.split_qkv(AO.linear(O.rms_norm(x, p.norm_w, 1e-5), p.qkv_w, p.qkv_b))
+    q, k = AO.rope(q, lengths), AO.rope(k, lengths)
+    o = []
+    for i, ((kc, vc), (ka, va)) in enumerate(zip(before, _held(cache, 1, tables))):
+        np.testing.assert_array_equal(ka[:-1], kc[:-1])   # the cached tokens stay
+        np.testing.assert_array_equal(va[:-1], vc[:-1])
+        kc[-1], vc[-1] = k[i], v[i]
+        oi, lse = AO.attention(q[i:i + 1], kc, vc, lengths[i:i + 1], 0)
+        o.append(AO.sink_scale(oi, lse, p.sinks))
+    y = AO.linear(np.concatenate(o).reshape(n, HQ * D), p.out_w, p.out_b)
+    close(got, O.f32_to_bf16(O.bf16_to_f32(x) + O.bf16_to_f32(y)))
+
+
+@pytest.mark.parametrize("n", sorted(_ROUTES))
+def test_attention_block_routes_prompt(A, attn_block, n):
+    """A short text of n tokens over 30 cached ones, through the same lines."""
+    from model.kv_cache import PagedKVCache
+    p, blk = attn_block
+    cache = PagedKVCache(num_layers=2, num_pages=12, max_batch=1, max_tokens=128)
+    cache.add_sequence(0)
+    cache.enable_sliding_window(0, 128)
+    x = O.make_input(59, 30 + n)
+    kc = np.zeros((0, HKV, D), dtype=np.uint16)
+    vc = kc.copy()
+    for a, b in ((0, 30), (30, 30 + n)):
+        cache.begin_forward([0], [b - a])
+        got = host_bf16(blk(bf16_dev(x[a:b]).view(1, b - a, 2880), cache).view(b - a, 2880))
+        cache.end_forward()
+        ref, k_new, v_new = AO.attn_block_forward(x[a:b], p, kc, vc, 0)
+        kc, vc = np.concatenate([kc, k_new]), np.concatenate([vc, v_new])
+        close(got, ref)
+
+
+@pytest.mark.parametrize("hidden,n,routes", [(3200, 16, (True, True)), (3200, 17, (False, True)),
+                                             (4104, 12, (False, True)), (4104, 50, (False, False)),
+                                             (192, 33, (True, True))])
+def test_attention_block_routes_row_sizes(A, hidden, n, routes):
+    """Hidden sizes past the fused QKV's limits (4096, above 16 tokens 3072) go
+    to the library from 9 tokens on; an output weight whose layout does not fit
+    does too, with the same result but for fp32 summation order."""
+    from model.attention import AttentionBlock
+    from model.config import GPTOssConfig
+    from model.kv_cache import PagedKVCache
+    p = AO.make_attn_params(62, hidden=hidden)
+    blk = AttentionBlock(GPTOssConfig(hidden_size=hidden), layer_idx=1, device="cuda")
+    for name, value in (("sinks", p.sinks), ("norm.weight", p.norm_w), ("qkv.weight", p.qkv_w),
+                        ("qkv.bias", p.qkv_b), ("out.weight", p.out_w), ("out.bias", p.out_b)):
+        blk.get_parameter(name).data.copy_(bf16_dev(value))
+    assert blk._fused(n) == routes
+    x = O.make_input(64, n, hidden=hidden)
+    none = np.zeros((0, HKV, D), dtype=np.uint16)
+    ref = AO.attn_block_forward(x, p, none, none, 0)[0]
+
+    def run():
+        cache = PagedKVCache(num_layers=2, num_pages=8, max_batch=1, max_tokens=128)
+        cache.add_sequence(0)
+        cache.enable_sliding_window(0, 128)
+        cache.begin_forward([0], [n])
+        return host_bf16(blk(bf16_dev(x).view(1, n, hidden), cache).view(n, hidden))
+
+    close(run(), ref)
+    blk.out.weight.data = blk.out.weight.data.t().contiguous().t()
+    assert blk._fused(n) == (routes[0], False)
+    close(run(), ref)
+
+
 def _ulp_close(got, ref, what, frac=0.01):
     """Equal but for fp32 summation order: at most `frac` of the elements
     differ, each by one bf16 ulp of its value, or -- for results near zero
