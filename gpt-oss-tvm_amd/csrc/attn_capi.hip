@@ -277,7 +277,7 @@ int check_gemv(const void* x, int64_t M, int64_t most, int64_t K, const void* W,
 
 // One token takes the vector-ALU GEMV (it streams W at the HBM's rate and its
 // sums need no second operand tile); from two tokens on its dot products bind
-// it (the unembedding at 5 tokens: 790 us against 192 at one), and the matrix
+// it (the unembedding at 5 tokens: 750 us against 188 at one), and the matrix
 // core form takes the call.
 int bias_residual(int64_t most, const uint16_t* x, int64_t M, int64_t K, const uint16_t* W,
                   int64_t N, const uint16_t* bias, const uint16_t* residual, uint16_t* out,

@@ -1,7 +1,8 @@
 // Dense projections of the gpt-oss layer for one token (dense_rows.hip takes
-// two and more): the fused QKV nn.Linear with its bias, YaRN RoPE and the KV-cache append; the
-// attention output nn.Linear with its bias and the residual add; the
-// unembedding (model/attention.py:204,254-256; model/transformer.py:95-100).
+// two and more): the fused QKV nn.Linear with its bias, YaRN RoPE and the
+// KV-cache append; the attention output nn.Linear with its bias and the residual
+// add; the unembedding (model/attention.py:204,254-256; model/transformer.py:
+// 95-100).
 // The QKV projection and the unembedding can also apply the RMSNorm before
 // them (attention.py:80, transformer.py:63) to the rows they stage.
 //

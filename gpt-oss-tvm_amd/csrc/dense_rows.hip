@@ -1,26 +1,27 @@
-// Dense projections for 2 to 16 token rows (the layers' two: to 64 and 48) on the bf16 matrix cores: the
-// fused QKV nn.Linear with its bias, YaRN RoPE and the KV-cache append; the
-// attention output nn.Linear with its bias and the residual add; the
-// unembedding (model/attention.py:204,254-256; model/transformer.py:95-100).
+// Dense projections for several token rows on the bf16 matrix cores: the fused QKV
+// nn.Linear with its bias, YaRN RoPE and the KV-cache append (2 to 64 tokens); the
+// attention output nn.Linear with its bias and the residual add (2 to 48); the
+// unembedding (2 to 8; model/attention.py:204,254-256; model/transformer.py:
+// 95-100).
 //
 // y[m][n] = sum_k t[m][k] W[n][k], bf16 operands, fp32 accumulation, one bf16
 // rounding, then the epilogue's own bf16 ops, as dense_gemv.hip (one token)
 // does.  Bound by the bytes of W: a vector dot product per (row, token) is
 // issue-bound from two tokens on, while the matrix cores multiply 16 W rows by
 // 16 tokens for the price of the loads: the 201088 x 2880 unembedding at 2, 5
-// and 8 tokens 399, 750 and 1122 us on the vector ALUs, 198-201 here (5.8 TB/s);
-// QKV with its norm at 2 and 8 tokens 19.1 and 54.1 us, 12.2-12.6 here; the output
-// projection 10.6 and 34.1, 7.1 here (rows_wide_kernel).  (One token stays on the
-// vector ALUs: 9.1 and 6.5 us.)
+// and 8 tokens 399, 750 and 1122 us on the vector ALUs, 198-206 here (5.6 to 5.8
+// TB/s); QKV with its norm at 2 and 8 tokens 19.1 and 54.1 us, 12.4-12.8 here; the
+// output projection 10.6 and 34.1, 7.1 here (rows_wide_kernel).  (One token stays on
+// the vector ALUs: unembedding 188 us against 205 here, QKV 9.1, output 6.5.)
 //
 // A workgroup takes 16 or 32 rows of W at a time; its sixteen waves split K
 // into contiguous runs of 32-wide steps (5 or 6 each at K = 2880), so that
 // every byte of the rows is in flight at once, and add their partial tiles
-// through LDS in fp64 (deterministic, one rounding).  v_mfma_f32_16x16x32_bf16: lane (r, g) =
-// (l % 16, l / 16) gives A row r (a W row) and B column r (a token), k = 8 g ..
-// 8 g + 7 of the step for both; D element i of the lane is W row 4 g + i,
-// token r.  Neither operand goes through LDS: a wave's K run of W and of the
-// tokens is used by that wave alone.
+// through LDS in fp64 (deterministic, one rounding).  v_mfma_f32_16x16x32_bf16:
+// lane (r, g) = (l % 16, l / 16) gives A row r (a W row) and B column r (a token),
+// k = 8 g .. 8 g + 7 of the step for both; D element i of the lane is W row
+// 4 g + i, token r.  Neither operand goes through LDS: a wave's K run of W and of
+// the tokens is used by that wave alone.
 // The tokens stay in registers (kSteps x 16 bytes a lane); for the unembedding a
 // workgroup walks a contiguous range of row groups with two groups' W in
 // flight.  The RMSNorm is the standalone kernel's arithmetic: the sum of squares
@@ -321,7 +322,8 @@ __global__ __launch_bounds__(kThreads) void rows_kernel(Args a) {
 // bytes a clock (QKV with its norm 15.1, 17.0, 21.3 and 24.2 us at 17, 32, 48 and
 // 64 tokens, output 10.9, 13.5, 17.5 and 21.4; so 13.2, 13.9, 16.1 and 17.8, output
 // 8.8, 9.5, 12.0 and 15.1; at 8 and 16 tokens 7.1 and 7.3, 8.9 and 10.3 in
-// rows_kernel's form).  Whole 128-byte lines per eight lanes changed nothing (13.6, 13.8, 15.6, 20.5; output 9.3, 9.7, 11.9, 14.7).  The partial tiles, fp32
+// rows_kernel's form).  Whole 128-byte lines per eight lanes were no better (13.6,
+// 13.8, 15.6 and 20.5; output 9.3, 9.7, 11.9 and 14.7).  The partial tiles, fp32
 // chains of at most 16 steps, are added over the waves in fp64 through LDS.  One
 // workgroup per CU: 180 (output) and 160 (QKV), one round.  The RMSNorm is its own
 // launch here (fused it would read the tokens twice).

@@ -108,20 +108,23 @@ class AttentionBlock(torch.nn.Module):
     def _fused(self, n: int) -> tuple[bool, bool]:
         """Whether n tokens take the fused QKV and output projections.  From 9
         tokens on the library's general form (any K, any weight layout) stays where
-        the fused kernels' limits do not hold.  Measured with norm and epilogues,
-        library / fused us: QKV at 16, 17, 48 and 64 tokens 19.3 / 13.4, 20.2 /
-        13.2, 21.8 / 16.1 and 24.5 / 17.8; output 14.2 / 7.3, 11.9 / 8.8, 12.8 /
-        12.0 and, past its limit of 48, 13.5 / 15.1."""
+        the fused kernels' limits do not hold.  A block of 9, 17, 48 and 64 decoding
+        sequences with up to 1000 keys (16 blocks in turn: weights from HBM), us with
+        both fused 33.0, 40.3, 50.1 and (output by the library) 58.2; with QKV by the
+        library 42.6, 49.0, 57.6 and 69.9; with the output 42.2, 44.7 and 51.6.  Past 48
+        tokens a fused output gains nothing: at 64, 1000 and 4096 keys, library 58.1 and
+        109.8, fused 57.1 and 109.5."""
         if n <= A.GEMV_MAX_TOKENS:
             return True, True
+        if n > A.ROWS_QKV_MAX_TOKENS:
+            return False, False
 
         def fits(w, most_k):
             return (w.shape[1] <= most_k and w.shape[1] % 8 == 0 and w.is_contiguous()
                     and w.data_ptr() % 16 == 0)
 
         wide = n > A.ROWS_NORM_MAX_TOKENS
-        return (n <= A.ROWS_QKV_MAX_TOKENS
-                and fits(self.qkv.weight, A.ROWS_WIDE_QKV_MAX_K if wide else 4096),
+        return (fits(self.qkv.weight, A.ROWS_WIDE_QKV_MAX_K if wide else 4096),
                 n <= A.ROWS_OUT_MAX_TOKENS and fits(self.out.weight, 4096))
 
     def _window(self, tables) -> int:

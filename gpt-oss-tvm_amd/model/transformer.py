@@ -11,8 +11,8 @@ loads through ``weights.TorchCheckpoint.load_into`` (embedding.weight,
 block.N.attn.*, block.N.mlp.*, norm.scale, unembedding.weight).
 
 Every operator is a HIP kernel of libmoe_gfx950; the dense bf16 projections
-(QKV, attention output, unembedding) are HIP GEMVs for up to 8 tokens and
-library GEMMs for more.
+are HIP kernels for few tokens (QKV up to 64, attention output 48, unembedding
+8) and library GEMMs for more.
 """
 from __future__ import annotations
 

@@ -42,7 +42,8 @@ MOE_API int attn_rms_norm(const uint16_t* x, int64_t n, int64_t H, const uint16_
  * output t @ W_qkv^T (model/attention.py:204, without its bias); this adds the
  * bias (a second bf16 rounding, nn.Linear), applies YaRN RoPE to q and k at
  * positions[i] (model/attention.py:94-178: inv_freq [32] fp32 and the
- * concentration 0.1 ln(factor) + 1 come from the caller), writes q [n, 64,
+ * concentration 0.1 ln(factor) + 1 come from the caller; angles positions[i] *
+ * inv_freq below 2^50, any YaRN table's, as in the fused forms), writes q [n, 64,
  * 64] bf16 to q_out and appends k and v at cache slot slots[i] = page * 16 +
  * offset (PagedKVCache.append_mha_kv, tvm_fix.patch:14-33).  Slots outside
  * [0, 16 num_pages) are not written. */
@@ -119,8 +120,9 @@ MOE_API int attn_embedding(const int32_t* ids, int64_t n, const uint16_t* table,
  * out[m][n] = bf16(sum_k t[m][k] W[n][k]), fp32 accumulation, one bf16
  * rounding, where t = x, or t = RMSNorm(x) with weight norm_w and eps when
  * norm_w is not NULL (the same arithmetic as attn_rms_norm; norm_w [K] may
- * begin at any element).  x [M, K], W [N, K], out [M, N] bf16; K % 8 == 0, K <= 4096.  Replaces the final norm and
- * the unembedding nn.Linear at decode (model/transformer.py:63,95-100). */
+ * begin at any element).  x [M, K], W [N, K], out [M, N] bf16; K % 8 == 0,
+ * K <= 4096.  Replaces the final norm and the unembedding nn.Linear at decode
+ * (model/transformer.py:63,95-100). */
 MOE_API int attn_gemv(const uint16_t* x, int64_t M, int64_t K, const uint16_t* W, int64_t N,
                       const uint16_t* norm_w, float eps, uint16_t* out, moe_stream_t stream);
 
