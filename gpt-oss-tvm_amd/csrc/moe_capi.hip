@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 
 #include "../../include/moe_gfx950.h"
 
@@ -97,26 +98,37 @@ inline size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 // Expert matmul dispatch (model/mlp_optimized.py:94-107 picks prefill or
 // decode kernels by token count): the tiled GEMM once the experts average 48 or
 // more pairs (each weight tile then serves many tokens); the grouped GEMV below
-// that or when N is not a multiple of the GEMM's tile.  With 64 or more experts
-// the block and its stages take the GEMM from 40 pairs on, above 128 tokens (what
-// the decode launch takes): there the GEMV's token batches overflow and it needs an
-// encoding pass besides.  Block us, GEMV / GEMM, at uniform routing and at Zipf
-// routing of beta 0.5 (the benchmark's) and 1.0:
-//   E = 64, 641 tokens (40.1 pairs)   417 / 364   412 / 391   402 / 379
-//           767 tokens (47.9)         495 / 382   446 / 409   423 / 421
-//   E = 128, 1280 tokens (40)         840 / 656   783 / 755   701 / 633
-//            1472 tokens (46)        1083 / 712   900 / 785   780 / 700
-// Fewer experts have units for a few rounds of workgroups only, and a last,
-// nearly empty round of the GEMM costs what the better tiles gain:
-//   E = 48, 528 tokens (44)           316 / 290   316 / 313   303 / 317
-//   E = 32, 328 tokens (41)           229 / 207   225 / 222   216 / 219
-//           383 tokens (47.9)         218 / 209   224 / 224   225 / 243
-//   E = 16, 168 tokens (42)           125 / 123   130 / 148   131 / 144
+// that or when N is not a multiple of the GEMM's tile.  Above 128 tokens (what the
+// decode launch takes) the block and its stages take the GEMM from 40 pairs on,
+// where the GEMV's token batches overflow and it needs an encoding pass besides,
+// if its rounds of workgroups are full: mlp1's units (96-row tiles, 48 pairs each)
+// run 512 at a time, and a last, nearly empty round costs what the better tiles
+// gain.  Skewed routing has the most units, about 0.72 part-filled tiles per expert
+// (Zipf of beta 0.75 to 1.2; 0.25 to 0.5 at uniform routing); past 5.5 rounds the
+// last one no longer matters.  Block us, GEMV / GEMM, at uniform routing and at Zipf
+// routing of beta 0.5 (the benchmark's) and 1.0, with the rounds at 0.72:
+//   E = 32, 322 tokens (40.3 pairs, 2.92)  219 / 189   222 / 218   215 / 214
+//           337 tokens (42.1, 3.00)        213 / 204   218 / 218   214 / 216
+//           383 tokens (47.9, 3.22)        215 / 208   222 / 223   222 / 239   no
+//   E = 40, 460 tokens (46, 3.93)          311 / 262   293 / 267   284 / 274
+//   E = 16, 168 tokens (42, 1.50)          125 / 123   130 / 148   131 / 144   no
+//   E = 48, 528 tokens (44, 4.60)          316 / 290   316 / 313   303 / 317   no
+//   E = 56, 561 tokens (40.1, 5.10)        335 / 321   339 / 350   335 / 349   no
+//           671 tokens (47.9, 5.64)        390 / 342   391 / 357   389 / 372
+//   E = 64, 641 tokens (40.1, 5.83)        417 / 364   412 / 391   402 / 379
+//           767 tokens (47.9, 6.44)        495 / 382   446 / 409   423 / 421
+//   E = 128, 1280 tokens (40, 11.6)        840 / 656   783 / 755   701 / 633
+//            1472 tokens (46, 12.6)       1083 / 712   900 / 785   780 / 700
 // One matmul alone saves no encoding pass: moe_einsum_fused stays with 48 (E = 64,
 // 680 tokens, bf16 rows, beta 1.0: 206 / 223).
 bool tiled_matmul(int64_t pairs, int64_t E) { return pairs >= 48 * E; }
-bool tiled_block(int64_t pairs, int64_t k, int64_t E) {
-  return tiled_matmul(pairs, E) || (E >= 64 && pairs > 128 * k && pairs >= 40 * E);
+bool full_rounds(int64_t pairs, int64_t E, int64_t I) {
+  const double rounds = ((double)pairs / 48 + 0.72 * (double)E) * (double)(2 * I / 192) / 512;
+  return rounds > 5.5 || (rounds <= 4 && rounds >= 0.96 * std::ceil(rounds));
+}
+bool tiled_block(int64_t pairs, int64_t k, int64_t E, int64_t I) {
+  return tiled_matmul(pairs, E) ||
+         (pairs > 128 * k && pairs >= 40 * E && full_rounds(pairs, E, I));
 }
 
 // The decode launch combines a token's k mlp2 rows itself (the last of its k
@@ -237,7 +249,7 @@ int mlp1_pieces(const void* t_pk, int64_t n, int64_t k, int64_t E, int64_t H, in
                 hipStream_t s) {
   const int nk = (int)(n * k);
   int rc;
-  const bool tiled = tiled_block(nk, k, E);
+  const bool tiled = tiled_block(nk, k, E, I);
   if (tiled && ((uintptr_t)bias & 15u) == 0) {
     rc = moe_launch_mx_gemm(t_pk, (int)n, kPiecesT, indptr, sp, (int)k, 0, 1, blocks, scales,
                             bias, (int)E, (int)(2 * I), (int)H, nk, 2, alpha, limit, act_pk,
@@ -401,7 +413,7 @@ int moe_mlp1_swiglu(const void* t_pieces, const int32_t* indptr, const int32_t* 
   if (!aligned16(t_pieces) || !aligned16(blocks) || ((uintptr_t)act & 3u)) return MOE_ERR_ALIGN;
   return expert_matmul(t_pieces, (int)n, kPiecesT, indptr, sorted_pairs, (int)k, 0, 1, blocks,
                        scales, bias, (int)E, (int)(2 * I), (int)H, (int)(n * k), (int)(n * k), 1,
-                       alpha, limit, act, (int)I, tiled_block(n * k, k, E), as_stream(stream));
+                       alpha, limit, act, (int)I, tiled_block(n * k, k, E, I), as_stream(stream));
 }
 
 int moe_mlp1_swiglu_pieces(const void* t_pieces, const int32_t* indptr,
@@ -432,7 +444,7 @@ int moe_mlp2(const void* act_pieces, const int32_t* indptr, const int32_t* sorte
   if (!aligned16(act_pieces) || !aligned16(blocks) || ((uintptr_t)y & 3u)) return MOE_ERR_ALIGN;
   return expert_matmul(act_pieces, (int)(n * k), kPiecesAct, indptr, sorted_pairs, (int)k, 2, 0,
                        blocks, scales, bias, (int)E, (int)H, (int)I, (int)(n * k), (int)(n * k), 0,
-                       0.f, 0.f, y, (int)H, tiled_block(n * k, k, E), as_stream(stream));
+                       0.f, 0.f, y, (int)H, tiled_block(n * k, k, E, I), as_stream(stream));
 }
 
 int moe_mlp_decode(const void* t_pieces, const int32_t* indptr, const int32_t* sorted_pairs,
@@ -540,7 +552,7 @@ static int block_forward_impl(const uint16_t* x, int64_t n, int64_t E, int64_t k
   float* logits = (float*)(ws + off[12]);
   int32_t* counts = (int32_t*)(ws + off[13]);
   int32_t* sync = (int32_t*)(ws + off[kRegionSync]);  // [E] counts, [E] status
-  const bool gemm = tiled_block(nk, k, E);
+  const bool gemm = tiled_block(nk, k, E, I);
   // norm, t, its pieces and the logits (and sync[0..E] = 0: the decode
   // launch's counts and status); then top-k, softmax and grouping
   void* t_qs = (char*)t_pk + moe_pieces_q_bytes(n, H, kPiecesT);

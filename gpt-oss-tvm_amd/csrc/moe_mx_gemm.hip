@@ -658,9 +658,11 @@ int launch_gm(int64_t rows_active, hipStream_t stream, const uint8_t* q, const u
 
 // Rows of a tile: 96 for mlp1 (two pieces, a SwiGLU epilogue) below 48 pairs per
 // expert on average (its 48 tokens then hold most experts), else 192.  Block us with
-// 96 / 192 rows, 128 experts at 1280, 1408 and 1535 tokens: uniform 656 / 688, 688 /
-// 701 and 720 / 713, Zipf routing of beta 0.5 755 / 768, 781 / 808 and 801 / 828, of
-// beta 1.0 633 / 646, 668 / 680 and 721 / 734.
+// 96 / 192 rows, at uniform routing and at Zipf routing of beta 0.5 and 1.0: 32
+// experts at 328 tokens 207 / 199, 222 / 222, 219 / 229 and at 336 tokens 209 / 196,
+// 222 / 227, 218 / 230; 128 experts at 1280 tokens 656 / 688, 755 / 768, 633 / 646
+// and at 1408 tokens 688 / 701, 781 / 808, 668 / 680: what 96 rows lose with few
+// experts at uniform routing they win with skewed ones.
 template <int P, int kEpi, class... A>
 int launch_rows(int64_t rows_active, int E, A... args) {
   if constexpr (P == 2 && kEpi >= 1)

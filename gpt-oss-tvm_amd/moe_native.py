@@ -257,8 +257,8 @@ def mlp1_swiglu_pieces(t_pieces, n, H, indptr, sorted_pairs, k, blocks, scales, 
     """mlp1 + SwiGLU -> act's three fp8 pieces (the block's prefill form).
 
     Returns (act_pieces, act): act [n*k, I] fp32 is scratch, written only when
-    the grouped GEMV runs (fewer than 48 pairs per expert on average; with 64 or
-    more experts and above 128 tokens fewer than 40).
+    the grouped GEMV runs (fewer than 48 pairs per expert on average; above 128
+    tokens fewer than 40, or units that leave a round of workgroups nearly empty).
     """
     E, N2, G, _ = blocks.shape
     inter = N2 // 2

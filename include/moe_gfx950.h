@@ -170,8 +170,9 @@ MOE_API int moe_mlp1_swiglu(const void* t_pieces, const int32_t* indptr,
  * mlp1 with the SwiGLU epilogue, its output act written as the three fp8 pieces
  * moe_mlp2 takes (moe_quantize_pieces(act, 1, n*k, I, 3), rows by sorted
  * position), as moe_block_forward runs it at prefill: with 48 or more pairs
- * per expert on average (64 or more experts, above 128 tokens: 40) the tiled
- * GEMM's epilogue encodes act directly (act is not written); below that the
+ * per expert on average (above 128 tokens 40, where the GEMM's units fill their
+ * rounds of workgroups) its epilogue encodes act directly (act is not written);
+ * else the
  * grouped GEMV writes act, fp32 [n*k, I] (caller-owned scratch), and the
  * encoding follows.
  * Replaces: mxfp4_moe_mlp1_prefill, model/mlp_optimized.py:214-351 (its bf16

@@ -637,19 +637,22 @@ def test_mlp1_swiglu_pieces(native, block20b, n, seed):
     assert np.array_equal(host_bf16(st2["out"]), host_bf16(st["out"]))
 
 
-@pytest.mark.parametrize("E,n,tiled", [(16, 176, False), (16, 191, False), (16, 192, True),
-                                       (32, 328, False), (32, 383, False), (63, 646, False),
-                                       (64, 639, False), (64, 640, True), (128, 1281, True)])
-def test_tiled_block_line(native, E, n, tiled):
-    """Where the block's GEMM begins: 48 pairs per expert on average, 40 from 64
-    experts on (fewer experts lose with skewed routing).  mlp1_swiglu_pieces
-    leaves its fp32 scratch as it was where the GEMM encodes act itself, and
-    the staged and the whole block agree bit for bit on either side."""
-    p = O.make_params(40 + E, num_experts=E, hidden=128, inter=96)
+@pytest.mark.parametrize("E,I,n,tiled", [
+    (16, 2880, 176, False), (16, 2880, 191, False), (16, 2880, 192, True),
+    (32, 2880, 319, False), (32, 2880, 320, True), (32, 2880, 337, True), (32, 2880, 338, False),
+    (32, 2880, 383, False), (32, 2880, 384, True), (40, 2880, 440, False), (40, 2880, 441, True),
+    (48, 2880, 575, False), (64, 2880, 639, False), (64, 2880, 640, True), (64, 96, 650, False),
+    (128, 2880, 1281, True)])
+def test_tiled_block_line(native, E, I, n, tiled):
+    """Where the block's GEMM begins: 48 pairs per expert on average, 40 where
+    mlp1's units fill their rounds of workgroups.  mlp1_swiglu_pieces leaves its
+    fp32 scratch as it was where the GEMM encodes act itself, and the staged and
+    the whole block agree bit for bit on either side."""
+    p = O.make_params(40 + E, num_experts=E, hidden=128, inter=I)
     blk = make_block(p)
     x = bf16_dev(O.make_input(41, n, hidden=128)).view(1, n, 128)
     st = blk.forward_staged(x)
-    act = torch.full((n * 4, 96), 12345.0, device="cuda")
+    act = torch.full((n * 4, I), 12345.0, device="cuda")
     _, act = native.mlp1_swiglu_pieces(
         native.quantize_pieces(st["t"], 2), n, 128, st["perm"]["indptr"],
         st["perm"]["sorted_pairs"], 4, blk.mlp1_weight_blocks, blk.mlp1_weight_scales,
@@ -662,16 +665,16 @@ def test_tiled_block_line(native, E, n, tiled):
                                                (16, 192, 96, 190, 92, True),
                                                (14, 128, 96, 140, 93, False),
                                                (13, 2880, 96, 150, 94, False),
-                                               (64, 384, 192, 660, 95, False),
-                                               (64, 192, 96, 760, 96, True),
-                                               (65, 128, 96, 652, 97, False),
-                                               (64, 2880, 96, 650, 98, False)])
+                                               (64, 384, 2880, 660, 95, False),
+                                               (64, 192, 2880, 760, 96, True),
+                                               (32, 128, 2880, 337, 97, False),
+                                               (32, 2880, 2880, 321, 98, False)])
 def test_block_gemm_small_tile(native, E, H, I, n, seed, skew):
-    """Above 128 tokens at 40 to 48 pairs per expert on average, fewer than 64
-    experts on the grouped GEMV, 64 and more with mlp1 on the GEMM's 96-row tile
-    (48 tokens): one, two, three and 23 chunks of K, one and two column tiles,
-    skewed routing (four experts of all tokens, the others without: 16 tiles
-    each with a ragged last one).  Act and output against the oracle."""
+    """Above 128 tokens at 40 to 48 pairs per expert on average: the first four on
+    the grouped GEMV (their units fill no round), the others with mlp1 on the
+    GEMM's 96-row tile (48 tokens): one, two, three and 23 chunks of K, skewed
+    routing (four experts of all tokens, the others without: 16 tiles each with a
+    ragged last one).  Act and output against the oracle."""
     p = O.make_params(seed, num_experts=E, hidden=H, inter=I)
     if skew:
         p.gate_b[:] = O.f32_to_bf16(np.array([10, 9, 8, 7] + [-10] * (E - 4), np.float32))
@@ -681,18 +684,6 @@ def test_block_gemm_small_tile(native, E, H, I, n, seed, skew):
 
 
 def test_mlp1_swiglu_pieces_small_tile(native, block20b):
-    """Act's pieces = quantize_pieces of its fp32 act, bit for bit, at 41 pairs
-    per expert of the 20B shape (the GEMV and the encoding pass)."""
+    """The 96-row tile's act pieces = quantize_pieces of its fp32 act, bit for
+    bit, at 41 pairs per expert of the 20B shape."""
     test_mlp1_swiglu_pieces(native, block20b, 328, 31)
-
-
-def test_mlp1_swiglu_pieces_96_rows(native):
-    """The same of the 96-row tile's epilogue: 64 experts of 41 pairs."""
-    p = O.make_params(45, num_experts=64, hidden=2880, inter=96)
-    blk, n = make_block(p), 656
-    x = bf16_dev(O.make_input(46, n)).view(1, n, 2880)
-    st = blk.forward_staged(x)
-    pk = blk.forward_staged(x, pieces_epilogue=True)["act_pieces"]
-    ref = PM.unpack(host(native.quantize_pieces(st["act"].contiguous(), 3)), n * 4, 96, 3)
-    for a, b in zip(PM.unpack(host(pk), n * 4, 96, 3), ref):
-        assert np.array_equal(a, b), np.argwhere(a != b)[:4]
